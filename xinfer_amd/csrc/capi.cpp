@@ -1,22 +1,24 @@
 // C ABI of libxinfer_attention_ops.so: validation, work planning and launches.
 //
 // The planner turns host-side lengths into a static schedule carried in the
-// kernel arguments (kernel_args.h): rows with at most 8 query vectors per KV
-// head go to the split-KV decode kernel, the others to the MFMA prefill
-// kernel; rows whose keys are split get fp32 partial records in the caller's
-// workspace, combined by a merge launch after the attention kernels or, for
-// small decode launches, by the last split of each (row, kv head) inside the
+// kernel arguments (kernel_args.h): rows with at most 32 query vectors per KV
+// head go to the decode kernel, the others to the MFMA prefill kernel; rows
+// whose keys are split get fp32 partial records in the caller's workspace,
+// combined by a merge launch after the attention kernels or, for decode rows
+// whose launch allows it, by the last split of each (row, kv head) inside the
 // decode launch (decode.hip: merge_in_launch), which folds in the merge
 // launch's order and arithmetic.  The schedule is a function of the shapes and
 // lengths only, never of tensor data, so results are deterministic and each
 // row is isolated from the others' contents.
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cmath>
 #include <cstdint>
 #include <cstdlib>
 #include <functional>
 #include <mutex>
+#include <numeric>
 #include <vector>
 
 #include "xinfer_attention.h"
@@ -26,17 +28,12 @@
 namespace xattn {
 namespace {
 
-constexpr int kDecodeMaxQueryVectors = 8;  // G * count at or below this: decode kernel
-constexpr int64_t kDecodeManyItems = 1536;  // one-round decode items from which items take several rounds
+constexpr int kCaptureDecodeMaxVectors = 8;  // graph capture: G * T at or below this takes the decode kernel
+constexpr int64_t kDecodeManyItems = 1536;  // one-pass decode items from which items are sized to the chip
 constexpr int kPrefillTileQ = 128;         // query vectors per prefill work item
 constexpr int64_t kPrefillMinSplitKeys = 512;
 
 int padded_dim(int64_t d) { return d <= 64 ? 64 : (d <= 128 ? 128 : 256); }
-int pow2_at_least(int x) {
-  int p = 1;
-  while (p < x) p <<= 1;
-  return p;
-}
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 struct Geometry {
@@ -72,11 +69,13 @@ int check_heads_and_dim(const Geometry &g) {
 struct Group {
   int row0 = 0, nrows = 0;
   AttnArgs dec{};
-  int dec_items = 0, dec_qr = 1, dec_rounds = 1;
+  int dec_items = 0, dec_columns = 1, dec_max_splits = 1;
   AttnArgs pre{};
   int pre_items = 0;
-  MergeArgs merge{};
-  int merge_items = 0, merge_max_splits = 0;
+  // Merge launches of the decode rows and of the prefill rows: their layouts
+  // differ (a thread folds a few splits, a row of lanes many).
+  MergeArgs dec_merge{}, pre_merge{};
+  int dec_merge_items = 0, pre_merge_items = 0, pre_max_splits = 1;
   // The decode launch may merge its split rows itself (decode_merge_fusable).
   bool dec_fusable = false;
 };
@@ -110,12 +109,12 @@ constexpr int kCusPerXcd = 32;
 // block wait, before it retires, for its record stores and one counter round
 // trip (kArrivalUs), which delays the blocks queued behind it once per wave of
 // resident blocks, and leaves the last split of each (row, kv head) a fold at
-// the tail (kInLaunchFoldUs).  Resident decode blocks: 256 CUs x 4 (the
-// kernels take 96-220 VGPRs per lane).
+// the tail (kInLaunchFoldUs).  Resident decode blocks: 256 CUs x 2 (64 KB of
+// each CU's 160 KB of LDS per block).
 constexpr double kDecodeMergeLaunchUs = 4.0;
 constexpr double kArrivalUs = 1.5;
 constexpr double kInLaunchFoldUs = 1.0;
-constexpr int64_t kDecodeResidentBlocks = 1024;
+constexpr int64_t kDecodeResidentBlocks = 512;
 // Decode kernel latency model: a launch floor, then whichever is longer of
 // streaming the KV bytes and the rounds of the items each resident block
 // runs one after another.
@@ -139,40 +138,72 @@ bool decode_merge_in_launch_pays(int64_t items) {
   return kArrivalUs * (double)ceil_div(items, kDecodeResidentBlocks) + kInLaunchFoldUs < kDecodeMergeLaunchUs;
 }
 
-// Rounds per decode item of rows [row0, row0 + nrows) (1 or
-// kDecodeItemRounds).  Launches with at least kDecodeManyItems one-round
-// items take kDecodeItemRounds: fewer, longer items cut the split records and
-// per-item work.  Smaller launches compare, by decode_launch_us, one-round
-// items against kDecodeItemRounds-round items when those bring every split
-// row within the in-launch merge (fusable: Hkv a multiple of 8 and no split
-// prefill row in the launch); longer items trade latency for the merge launch.
-// Measured on MI355X (cfg3 seeds 1 and 3, one round + merge launch against
-// four rounds + in-launch merge): 10.2 / 11.9 us and 13.6 / 12.8 us; the
-// model picks the faster of each.
-int choose_decode_rounds(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths,
-                         int64_t row0, int nrows, int G, int dp, int qr, bool fusable) {
-  int64_t items[2] = {0, 0}, max_splits[2] = {1, 1};
-  double kv_bytes = 0;
+// Keys per decode item of rows [row0, row0 + nrows), in whole passes of a
+// block's four waves (decode_tokens_per_item).
+//
+// Launches with at least kDecodeManyItems one-pass items, and those with rows of
+// more than kExactVectors query vectors (whose records are large) or beside
+// prefill rows, size their items to the chip (sized; kernel_args.h: kDecodeCus).
+// Smaller launches compare, by decode_launch_us, items of one pass against items
+// of kDecodeItemRounds passes when those bring every split row within eight
+// splits (fusable: Hkv a multiple of 8 and no split prefill row in the launch);
+// longer items trade latency for the merge launch.  Measured on MI355X (cfg3
+// seeds 1 and 3, one pass + merge launch against four passes + in-launch merge):
+// 10.2 / 11.9 us and 13.6 / 12.8 us; the model picks the faster of each.
+// vectors: rows of up to that many query vectors per KV head are decode rows.
+struct DecodeChoice {
+  bool sized;
+  int64_t keys;
+};
+DecodeChoice choose_decode(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths,
+                           int64_t row0, int nrows, int G, int dp, int64_t vectors, bool fusable) {
+  int64_t items[2] = {0, 0}, max_splits[2] = {1, 1}, keys = 0, widest = 0, longest = 1, pairs = 0;
+  bool prefill = false;
+  const int64_t pass = decode_tokens_per_item(dp);
   const int rounds[2] = {1, kDecodeItemRounds};
+  std::array<int64_t, kMaxRows> passes;
+  int n = 0;
   for (int r = 0; r < nrows; ++r) {
     const int64_t qv = (int64_t)counts[row0 + r] * G, len = lengths[row0 + r];
-    if (qv <= 0 || qv > kDecodeMaxQueryVectors) continue;
-    kv_bytes += 4.0 * (double)(len * g.Hkv * g.D);
+    prefill = prefill || qv > vectors;
+    if (qv <= 0 || qv > vectors) continue;
+    widest = std::max(widest, qv);
+    keys += g.Hkv * len;
+    pairs += g.Hkv;
+    passes[n++] = ceil_div(len, pass);
+    longest = std::max(longest, ceil_div(len, pass));
     for (int o = 0; o < 2; ++o) {
-      const int64_t splits = ceil_div(len, rounds[o] * decode_tokens_per_item(dp, qr));
+      const int64_t splits = ceil_div(len, rounds[o] * pass);
       items[o] += g.Hkv * splits;
       max_splits[o] = std::max(max_splits[o], splits);
     }
   }
-  if (items[0] >= kDecodeManyItems) return kDecodeItemRounds;
-  if (!fusable || max_splits[1] > kMergeSerialSplits) return 1;
+  if (items[0] >= kDecodeManyItems || widest > kExactVectors || prefill) {
+    // The fewest passes per item that leave at most `limit` items.
+    auto least = [&](int64_t limit) {
+      int64_t m = std::max<int64_t>(1, ceil_div(items[0], limit));
+      for (; m < longest; ++m) {
+        int64_t count = 0;
+        for (int r = 0; r < n; ++r) count += g.Hkv * ceil_div(passes[r], m);
+        if (count <= std::max(limit, pairs)) break;
+      }
+      return m;
+    };
+    auto even = [&](int64_t m, int64_t limit) { return m * limit * kDecodeEvenDen <= items[0] * kDecodeEvenNum; };
+    const int64_t m1 = least(kDecodeCus), m2 = least(2 * kDecodeCus);
+    int64_t m = 2 * m2 < m1 ? m2 : m1;
+    if (!even(m1, kDecodeCus) && !even(m2, 2 * kDecodeCus)) m = least(4 * kDecodeCus);
+    return {true, m * pass};
+  }
+  if (!fusable || max_splits[1] > kMergeSerialSplits) return {false, pass};
+  const double kv_bytes = 4.0 * (double)(keys * g.D);
   double us[2];
   for (int o = 0; o < 2; ++o) {
     const bool split = max_splits[o] > 1;
     const bool in_launch = max_splits[o] <= kMergeSerialSplits && decode_merge_in_launch_pays(items[o]);
     us[o] = decode_launch_us(items[o], rounds[o], kv_bytes, split, in_launch);
   }
-  return us[1] < us[0] ? kDecodeItemRounds : 1;
+  return {false, (us[1] < us[0] ? kDecodeItemRounds : 1) * pass};
 }
 
 // 64-key tiles of prefill item (split, query tile) of row rs: the key range
@@ -257,12 +288,12 @@ int32_t prefill_splits(int64_t len, int64_t split_keys) {
 // their time (total work over 256 CUs, or the longest item, plus the
 // records), until that bound passes the best time found.
 int64_t choose_split_keys(const Geometry &g, const std::vector<int32_t> &counts,
-                          const std::vector<int32_t> &lengths, int G, int dp) {
+                          const std::vector<int32_t> &lengths, int G, int dp, int64_t decode_vectors) {
   int64_t prefill_keys = 0;
   std::vector<RowSched> rows;
   for (int64_t r = 0; r < g.B; ++r) {
     const int64_t qv = (int64_t)counts[r] * G;
-    if (qv <= kDecodeMaxQueryVectors) continue;
+    if (qv <= decode_vectors) continue;
     prefill_keys += g.Hkv * ceil_div(qv, kPrefillTileQ) * lengths[r];
     RowSched rs{};
     rs.count = counts[r];
@@ -353,17 +384,15 @@ int64_t choose_split_keys(const Geometry &g, const std::vector<int32_t> &counts,
   return best_keys;
 }
 
-// Whether a group's decode launch can merge its own split rows: it has split
-// decode rows and no split prefill row (whose records need the merge launch
-// anyway), every split row has at most kMergeSerialSplits splits (the merge
-// layout the in-launch fold reproduces), and Hkv is a multiple of 8 (the
-// kernel gives XCD x the kv heads h = x mod 8 of every row).
+// Whether a group's decode launch can merge its own split rows: Hkv is a
+// multiple of 8 (the kernel gives XCD x the kv heads h = x mod 8 of every row),
+// and every split row has at most kMergeSerialSplits splits, the merge layout
+// the in-launch fold reproduces.  More splits, or vectors, make the fold at the
+// launch's tail longer than a merge launch, which spreads it over the chip
+// (measured on MI355X: 12 vectors of up to 11 splits 53.8 us against 29.5 + 4.6,
+// 2 vectors of up to 12 splits 28.4 against 22.8 + 4.5).
 bool decode_merge_fusable(const Group &grp, int64_t Hkv) {
-  if (grp.dec_items == 0 || grp.merge_items == 0 || Hkv % 8 != 0) return false;
-  if (grp.merge_max_splits > kMergeSerialSplits) return false;
-  for (int r = 0; r < grp.pre.nrows; ++r)
-    if (grp.pre.rows[r].nsplit > 1) return false;
-  return true;
+  return grp.dec_items > 0 && grp.dec_merge_items > 0 && Hkv % 8 == 0 && grp.dec_max_splits <= kMergeSerialSplits;
 }
 
 // Whether this device deals consecutive blocks to its 8 XCDs in turn, probed
@@ -407,10 +436,34 @@ bool merge_launch_forced() {
   return forced;
 }
 
-// A nonzero tag below 2^36 for every decode launch with the in-launch merge.
+// A nonzero tag below 2^36 for every decode launch that counts arrivals; not a
+// small number, which other data left in the workspace may look like.
 uint64_t next_launch_tag() {
   static std::atomic<uint64_t> sequence{0};
-  return sequence.fetch_add(1, std::memory_order_relaxed) % ((uint64_t(1) << 36) - 1) + 1;
+  constexpr uint64_t kTags = (uint64_t(1) << 36) - 1;  // no common factor with the step below
+  return sequence.fetch_add(1, std::memory_order_relaxed) % kTags * 0x5851f45ull % kTags + 1;
+}
+
+// Query vectors per KV head up to which a row of the call takes the decode
+// kernel: kStreamMaxVectors, whose columns hold them and whose stream is bound by
+// HBM; but kExactVectors, as far as the weights' precision needs it, where a
+// decode launch would serve only a few keys of rows with more beside prefill
+// rows.  Measured on MI355X: prompts of 77, 201 and 13 tokens (one vector each,
+// D = 64) 13.4 us in one launch, 17.6 with the 13-token row in its own; eight rows
+// of 2-6 tokens (12 vectors) over 39000 keys 73 us with the prefill kernel's
+// 128-vector tiles, 36 with this one.
+constexpr int64_t kShortRowKeys = 32768;  // keys of all KV heads
+int64_t decode_vector_limit(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths,
+                            int G) {
+  bool narrow = false, wide = false;
+  int64_t keys = 0;
+  for (int64_t r = 0; r < g.B; ++r) {
+    const int64_t qv = (int64_t)counts[r] * G;
+    if (qv > kStreamMaxVectors) wide = true;
+    else if (qv > kExactVectors) keys += g.Hkv * lengths[r];
+    else if (qv > 0) narrow = true;
+  }
+  return wide && !narrow && keys <= kShortRowKeys ? kExactVectors : kStreamMaxVectors;
 }
 
 // counts/lengths: per-row real queries and populated KV lengths (validated).
@@ -420,28 +473,28 @@ Plan make_plan(const Geometry &g, const std::vector<int32_t> &counts, const std:
   const int G = (int)(g.Hq / g.Hkv);
   const int dp = padded_dim(g.D);
 
+  const int64_t decode_vectors = decode_vector_limit(g, counts, lengths, G);
   // Keys per prefill split, chosen from the whole call's prefill work.
-  const int64_t split_keys = choose_split_keys(g, counts, lengths, G, dp);
+  const int64_t split_keys = choose_split_keys(g, counts, lengths, G, dp, decode_vectors);
 
   for (int64_t row0 = 0; row0 < g.B; row0 += kMaxRows) {
     Group grp;
     grp.row0 = (int)row0;
     grp.nrows = (int)std::min<int64_t>(kMaxRows, g.B - row0);
-    int max_qv = 1;
-    for (int r = 0; r < grp.nrows; ++r) {
-      const int qv = counts[row0 + r] * G;
-      if (qv > 0 && qv <= kDecodeMaxQueryVectors) max_qv = std::max(max_qv, qv);
-    }
-    grp.dec_qr = pow2_at_least(max_qv);
     bool prefill_split = false;
     for (int r = 0; r < grp.nrows; ++r) {
       const int64_t qv = (int64_t)counts[row0 + r] * G;
-      if (qv > kDecodeMaxQueryVectors && prefill_splits(lengths[row0 + r], split_keys) > 1) prefill_split = true;
+      if (qv > decode_vectors && prefill_splits(lengths[row0 + r], split_keys) > 1) prefill_split = true;
     }
-    grp.dec_rounds = choose_decode_rounds(g, counts, lengths, row0, grp.nrows, G, dp, grp.dec_qr,
-                                          g.Hkv % 8 == 0 && !prefill_split);
-    const int tpi = grp.dec_rounds * decode_tokens_per_item(dp, grp.dec_qr);
-    for (int r = 0; r < grp.nrows; ++r) {
+    const DecodeChoice choice = choose_decode(g, counts, lengths, row0, grp.nrows, G, dp, decode_vectors,
+                                              g.Hkv % 8 == 0 && !prefill_split);
+    int64_t records = 0;  // of this group: the groups' launches run one after another
+    // Longer rows first: the launch's last items are then short ones.
+    std::vector<int> order(grp.nrows);
+    std::iota(order.begin(), order.end(), 0);
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int x, int y) { return lengths[row0 + x] > lengths[row0 + y]; });
+    for (const int r : order) {
       const int64_t b = row0 + r;
       const int cnt = counts[b], len = lengths[b];
       const int64_t qv = (int64_t)cnt * G;
@@ -451,36 +504,45 @@ Plan make_plan(const Geometry &g, const std::vector<int32_t> &counts, const std:
       rs.length = len;
       rs.ntiles = 1;
       rs.nsplit = 1;
-      const bool decode = qv <= kDecodeMaxQueryVectors;  // includes rows with no query (zero fill only)
+      const bool decode = qv <= decode_vectors;  // includes rows with no query (zero fill only)
       if (decode) {
-        if (cnt > 0) rs.nsplit = (int32_t)ceil_div(len, tpi);
+        grp.dec_columns = std::max(grp.dec_columns, decode_column_groups((int)qv));
+        if (cnt > 0) rs.nsplit = (int32_t)ceil_div(len, choice.keys);
+        // Equal splits, in whole wave tiles: none is empty, since a split never
+        // holds more than choice.keys, a multiple of them.
+        const int64_t tile = decode_tokens_per_item(dp) / kDecodeWaves;
+        rs.ntiles = (int32_t)(ceil_div(ceil_div(len, rs.nsplit), tile) * tile);
         rs.item_begin = grp.dec_items;
         grp.dec_items += (int)(g.Hkv * rs.nsplit);
+        grp.dec_max_splits = std::max(grp.dec_max_splits, (int)rs.nsplit);
       } else {
         rs.ntiles = (int32_t)ceil_div(qv, kPrefillTileQ);
         rs.nsplit = prefill_splits(len, split_keys);
         rs.item_begin = grp.pre_items;
         grp.pre_items += (int)(g.Hkv * rs.ntiles * rs.nsplit);
+        grp.pre_max_splits = std::max(grp.pre_max_splits, (int)rs.nsplit);
       }
       if (rs.nsplit > 1) {
         // Decode: [kv head][split][vector] records.  Prefill: per (kv head,
         // split, query tile) a block of kPrefillTileQ records.
-        rs.rec_begin = plan.records;
-        plan.records += g.Hkv * rs.nsplit * (decode ? qv : rs.ntiles * kPrefillTileQ);
-        MergeRow &mr = grp.merge.rows[grp.merge.nrows++];
+        rs.rec_begin = records;
+        records += g.Hkv * rs.nsplit * (decode ? qv : rs.ntiles * kPrefillTileQ);
+        MergeArgs &merge = decode ? grp.dec_merge : grp.pre_merge;
+        int &merge_items = decode ? grp.dec_merge_items : grp.pre_merge_items;
+        MergeRow &mr = merge.rows[merge.nrows++];
         mr.batch = (int32_t)b;
         mr.count = cnt;
         mr.nsplit = rs.nsplit;
-        mr.item_begin = grp.merge_items;
+        mr.item_begin = merge_items;
         mr.tiles = decode ? 0 : rs.ntiles;
         mr.rec_begin = rs.rec_begin;
-        grp.merge_items += (int)(g.Hkv * qv);
-        grp.merge_max_splits = std::max(grp.merge_max_splits, (int)rs.nsplit);
+        merge_items += (int)(g.Hkv * qv);
       }
       AttnArgs &a = decode ? grp.dec : grp.pre;
       a.rows[a.nrows++] = rs;
     }
-    grp.dec_fusable = decode_merge_fusable(grp, g.Hkv);
+    plan.records = std::max(plan.records, records);
+    grp.dec_fusable = decode_merge_fusable(grp, g.Hkv) && !(prefill_split && !choice.sized);
     if (grp.dec_fusable) plan.counters = std::max<int64_t>(plan.counters, grp.dec_items);
     if (grp.pre_items > 0) xcd_runs(prefill_item_work(grp.pre.rows, grp.pre.nrows, g.Hkv, G, dp), grp.pre.xcd_begin);
     plan.groups.push_back(grp);
@@ -561,13 +623,15 @@ int run_plan(const Plan &plan, const Geometry &g, const xinfer_view4 &q, const x
         xcd_dispatch_round_robin(stream)) {
       grp.dec.arrive_ctr = reinterpret_cast<uint64_t *>(static_cast<char *>(workspace) + plan.counters_offset());
       grp.dec.tag = next_launch_tag();
-      grp.merge_items = 0;  // every split row is a decode row, merged in the launch
+      grp.dec_merge_items = 0;  // the decode rows are merged in the launch
     }
-    if (grp.dec_items > 0 && launch_decode(grp.dec, dp, grp.dec_qr, grp.dec_rounds, grp.dec_items, stream) != hipSuccess)
+    if (grp.dec_items > 0 && launch_decode(grp.dec, dp, grp.dec_columns, grp.dec_items, stream) != hipSuccess)
       return XINFER_ERR_LAUNCH;
     if (grp.pre_items > 0 && launch_prefill(grp.pre, dp, stream) != hipSuccess) return XINFER_ERR_LAUNCH;
-    if (grp.merge_items > 0) {
-      MergeArgs &m = grp.merge;
+    for (const bool decode : {true, false}) {
+      MergeArgs &m = decode ? grp.dec_merge : grp.pre_merge;
+      m.total_items = decode ? grp.dec_merge_items : grp.pre_merge_items;
+      if (m.total_items == 0) continue;
       m.out = static_cast<uint16_t *>(const_cast<void *>(out.data));
       m.o_sb = out.stride[0];
       m.o_sh = out.stride[1];
@@ -576,8 +640,8 @@ int run_plan(const Plan &plan, const Geometry &g, const xinfer_view4 &q, const x
       m.part_ml = part_ml;
       m.D = (int32_t)g.D;
       m.G = G;
-      m.total_items = grp.merge_items;
-      if (launch_merge(m, dp, grp.merge_max_splits, stream) != hipSuccess) return XINFER_ERR_LAUNCH;
+      if (launch_merge(m, dp, decode ? grp.dec_max_splits : grp.pre_max_splits, stream) != hipSuccess)
+        return XINFER_ERR_LAUNCH;
     }
   }
   return XINFER_OK;
@@ -650,11 +714,11 @@ int check_batched(const xinfer_view4 *q, const xinfer_view4 *k, const xinfer_vie
 
 // Graph-capture mode (xinfer_batched_flash_attention_graph): a plan that
 // depends only on the shapes.  Rows must take the decode kernel (at most
-// kDecodeMaxQueryVectors query vectors per KV head, i.e. T * G <= 8) and fit
+// kCaptureDecodeMaxVectors query vectors per KV head, i.e. T * G <= 8) and fit
 // one row table (B <= kMaxRows, which the kernels' per-block tables assume).
 // Records are laid out for every row at capacity.
 struct CapturePlan {
-  int dp = 0, qr = 1, rounds = 1, tok_item = 0, splits_max = 0, decode_blocks = 0;
+  int dp = 0, columns = 1, splits_max = 0, decode_blocks = 0, pass_min = 1;
   int64_t row_records = 0, records = 0;
   int64_t dp_d = 0;  // the head dim D (records hold D floats)
   // Prefill shapes (T * Hq/Hkv > 8): every row takes the prefill kernel,
@@ -668,13 +732,10 @@ struct CapturePlan {
   size_t merge_offset() const { return attn_offset() + (sizeof(AttnArgs) + 255) / 256 * 256; }
   size_t bytes() const { return prefill ? merge_offset() + sizeof(MergeArgs) : records_bytes(); }
 };
-// Decode blocks of a capture launch: every item of the capacity layout, at
-// most eight per CU of the 256.  With one-round items the blocks take the
-// valid items in turn; multi-round items (kDecodeItemRounds rounds, chosen
-// when the capacity layout has as many one-round items as the default
-// planner's threshold and its multi-round items fit this grid) take one block
-// each.
-constexpr int kCaptureMaxBlocks = 2048;
+// A decode launch's records are sized for items of kDecodeItemRounds passes
+// where the capacity layout has at least kCaptureManyItems items of one pass and
+// at most kCaptureItems of the longer ones; else for items of one pass.
+constexpr int64_t kCaptureManyItems = 1536, kCaptureItems = 2048;
 
 int check_capture(const xinfer_view4 *q, const xinfer_view4 *k, const xinfer_view4 *v, Geometry &g,
                   CapturePlan &cp) {
@@ -689,7 +750,7 @@ int check_capture(const xinfer_view4 *q, const xinfer_view4 *k, const xinfer_vie
   if (g.B > kMaxRows) return XINFER_ERR_CAPTURE_ROWS;
   cp.dp = padded_dim(g.D);
   cp.dp_d = g.D;
-  if (g.T * G > kDecodeMaxQueryVectors) {
+  if (g.T * G > kCaptureDecodeMaxVectors) {
     // Prefill shapes: the device plan (prefill.hip:
     // prefill_capture_plan_kernel) picks the split size from the lengths, in
     // the range choose_split_keys searches, so that the items stay below
@@ -708,16 +769,17 @@ int check_capture(const xinfer_view4 *q, const xinfer_view4 *k, const xinfer_vie
       return XINFER_ERR_QKV_SHAPES;
     return XINFER_OK;
   }
-  cp.qr = pow2_at_least((int)std::max<int64_t>(1, g.T * G));
-  const int tok_round = decode_tokens_per_item(cp.dp, cp.qr);
+  cp.columns = decode_column_groups((int)(g.T * G));
+  const int tok_round = decode_tokens_per_item(cp.dp);
   const int64_t one_round_items = g.B * g.Hkv * ceil_div(g.C, tok_round);
   const int64_t multi_round_items = g.B * g.Hkv * ceil_div(g.C, (int64_t)kDecodeItemRounds * tok_round);
-  cp.rounds = one_round_items >= kDecodeManyItems && multi_round_items <= kCaptureMaxBlocks ? kDecodeItemRounds : 1;
-  cp.tok_item = cp.rounds * tok_round;
-  cp.splits_max = (int)ceil_div(g.C, cp.tok_item);
-  cp.row_records = g.Hkv * cp.splits_max * g.T * G;
-  cp.records = cp.splits_max > 1 ? g.B * cp.row_records : 0;
-  cp.decode_blocks = (int)std::min<int64_t>(std::max<int64_t>(1, g.B * g.Hkv * cp.splits_max), kCaptureMaxBlocks);
+  const int rounds = one_round_items >= kCaptureManyItems && multi_round_items <= kCaptureItems ? kDecodeItemRounds : 1;
+  cp.pass_min = rounds;
+  cp.splits_max = (int)ceil_div(g.C, rounds * tok_round);
+  const int64_t pairs = g.B * g.Hkv, vectors = g.T * G;
+  cp.records = cp.splits_max > 1 ? pairs * cp.splits_max * vectors : 0;
+  // Every item the kernel may lay out (device_common.h: capture_splits).
+  cp.decode_blocks = (int)(ceil_div(std::min<int64_t>(pairs * cp.splits_max, 4 * kDecodeCus + pairs), 8) * 8);
   return XINFER_OK;
 }
 
@@ -840,11 +902,8 @@ int xinfer_batched_flash_attention_graph(const xinfer_view4 *q, const xinfer_vie
   c.T = (int32_t)g.T;
   c.B = (int32_t)g.B;
   c.C = (int32_t)g.C;
-  c.tok_item = cp.tok_item;
-  c.row_records = cp.row_records;
   c.blocks = blocks;
   c.blocks_stride = blocks_stride;
-  c.total_items = (int32_t)(g.B * g.Hkv * cp.splits_max);
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (cp.prefill) {
     char *ws = static_cast<char *>(workspace);
@@ -866,11 +925,13 @@ int xinfer_batched_flash_attention_graph(const xinfer_view4 *q, const xinfer_vie
       return XINFER_ERR_LAUNCH;
     return XINFER_OK;
   }
-  if (launch_decode_capture(c, cp.dp, cp.qr, cp.rounds, cp.decode_blocks, s) != hipSuccess) return XINFER_ERR_LAUNCH;
-  if (cp.splits_max > 1) {
-    c.total_items = (int32_t)(g.B * g.Hkv * g.T * c.G);
-    if (launch_merge_capture(c, cp.dp, cp.splits_max, s) != hipSuccess) return XINFER_ERR_LAUNCH;
-  }
+  c.pass_keys = decode_tokens_per_item(cp.dp);
+  c.pass_min = cp.pass_min;
+  c.splits_max = cp.splits_max;
+  c.row_records = g.Hkv * cp.splits_max * g.T * c.G;
+  if (launch_decode_capture(c, cp.dp, cp.columns, cp.decode_blocks, s) != hipSuccess) return XINFER_ERR_LAUNCH;
+  if (cp.splits_max > 1 && launch_merge_capture(c, cp.dp, s) != hipSuccess)
+    return XINFER_ERR_LAUNCH;
   return XINFER_OK;
 }
 

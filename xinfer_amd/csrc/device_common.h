@@ -249,12 +249,48 @@ __device__ __forceinline__ int read_page(const int32_t *blocks, int64_t stride, 
 }
 __device__ __forceinline__ int page_in_range(int page, int rows) { return min(max(page, 0), rows - 1); }
 
+// Inclusive prefix sum over the 64 lanes (DPP row shifts, then row broadcasts).
+__device__ __forceinline__ int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, true);  // row_bcast:15 into rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, true);  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+__device__ __forceinline__ int wave_total(int x) { return __builtin_amdgcn_readlane(wave_scan(x), 63); }
+
 // Row r's query count and KV length from the device offsets, clamped to the
 // ranges the host validates in the default mode (see CaptureArgs in kernel_args.h).
 __device__ __forceinline__ void capture_row(const CaptureArgs &c, int r, int &count, int &length) {
   const int32_t *cuq = c.offsets, *cuk = c.offsets + c.B + 1;
   count = min(max(cuq[r + 1] - cuq[r], 0), min(c.T, c.C));
   length = min(max(cuk[r + 1] - cuk[r], max(count, 1)), c.C);
+}
+
+
+// Splits of row `lane` of a graph-capture decode launch (every lane of the wave
+// calls it): the host planner's choice (capi.cpp: choose_decode) from the
+// device lengths, with a coarser search.  Items take whole passes of a block, at
+// least c.pass_min; there are never more than 4 * kDecodeCus + the (row, kv head)
+// pairs, and no row takes more than c.splits_max splits (the records hold those).
+__device__ __forceinline__ int capture_splits(const CaptureArgs &c, int lane, int count, int length) {
+  const bool active = lane < c.B && count > 0;
+  const int passes = active ? (length + c.pass_keys - 1) / c.pass_keys : 0;
+  const int total = c.Hkv * wave_total(passes);
+  // The fewest passes per item that leave at most `limit` items, up to one past
+  // the most that keep `limit` items about even.
+  auto most = [&](int limit) { return (int)((int64_t)total * kDecodeEvenNum / (limit * kDecodeEvenDen)) + 1; };
+  auto least = [&](int limit, int up_to) {
+    int m = max(c.pass_min, (total + limit - 1) / limit);
+    while (m < up_to && c.Hkv * wave_total((passes + m - 1) / m) > limit) m += 1 + m / 8;
+    return m;
+  };
+  const int m1 = least(kDecodeCus, most(kDecodeCus)), m2 = least(2 * kDecodeCus, most(2 * kDecodeCus));
+  int m = 2 * m2 < m1 ? m2 : m1;
+  if (m1 >= most(kDecodeCus) && m2 >= most(2 * kDecodeCus)) m = least(4 * kDecodeCus, most(kDecodeCus));
+  return active ? min((passes + m - 1) / m, c.splits_max) : 1;
 }
 
 }  // namespace xattn

@@ -18,7 +18,7 @@ struct RowSched {
   int32_t length;       // populated KV length after the append (>= count, >= 1)
   int32_t item_begin;   // first work item (blockIdx.x) of this row
   int32_t nsplit;       // KV splits per group; 1 = no partial records
-  int32_t ntiles;       // query tiles per kv head (prefill); 1 for decode
+  int32_t ntiles;       // query tiles per kv head (prefill); keys of one split (decode)
   int64_t rec_begin;    // first partial record of this row in the workspace
 };
 // Strided bf16 rank-4 tensor: element pointer + strides of dims 0..2 (dim 3 is unit).
@@ -79,27 +79,40 @@ struct MergeArgs {
   MergeRow rows[kMaxRows];
 };
 
-// Graph-capture decode (decode.hip, merge.hip): one launch shape serves every
-// step, because the kernels read each row's query count and KV length from
-// the device copy of the cumulative offsets instead of a host schedule.
-// Records are laid out per row at capacity: row r's start at r * row_records,
-// in the decode layout [kv head][split][vector] with the row's actual split
-// count.  Counts are clamped to [0, min(T, C)] and lengths to [max(count, 1), C], so
-// no device data can address outside q, k, v, out or the workspace.
+// Graph-capture mode: one launch shape serves every step, because the kernels
+// read each row's query count and KV length from the device copy of the
+// cumulative offsets instead of a host schedule.  Counts are clamped to
+// [0, min(T, C)] and lengths to [max(count, 1), C], so no device data can
+// address outside q, k, v, out or the workspace.
 struct CaptureArgs {
   View q, k, v;
   uint16_t *out;             // contiguous [B, Hq, T, D]
   int64_t o_sb, o_sh, o_st;
-  float *part_o, *part_ml;   // records of every row at capacity
+  float *part_o, *part_ml;   // split records
   const int32_t *offsets;    // device [2][B + 1]: cumulative counts, cumulative lengths
   float scale_log2;
   int32_t D, G, Hkv, T, B, C;
-  int32_t tok_item;          // keys per decode work item
-  int32_t total_items;       // decode: items at capacity; merge: query vectors at capacity
-  int64_t row_records;       // records per row at capacity: Hkv * ceil(C / tok_item) * T * G
   const int32_t *blocks;     // page table as in AttnArgs (nullable), over the B rows of k/v
   int64_t blocks_stride;
+  // Decode: row r's records start at r * row_records, [kv head][split][vector]
+  // with the row's splits (device_common.h: capture_splits).
+  int64_t row_records;
+  int32_t pass_keys;         // keys a block's waves take together
+  int32_t pass_min;          // least passes per item
+  int32_t splits_max;        // most splits of a row
 };
+
+// Decode items for a launch that fills the chip: one per CU or two, whichever
+// leaves the longest item closer to a CU's (half a CU's) even share of the keys;
+// at most four per CU if both leave it more than kDecodeEvenNum / kDecodeEvenDen
+// of that share.  A CU reads at most about 45 GB/s, 1.8 times its share of HBM, so
+// what counts is that every CU gets about the same bytes.  Measured on MI355X
+// (decode kernel, items of 128-key passes, D = 128): 126 MB of KV 22.8 us with 512
+// items (two on every CU), 22.8 with 240 (one), 27.9 with 312 and 25.5 with 280
+// (some CUs hold two); 226 MB in 32 rows, 24 of them short, 41.2 with 1008 items,
+// 45.8 with 512, 49.9 with 456.
+constexpr int kDecodeCus = 256;
+constexpr int kDecodeEvenNum = 7, kDecodeEvenDen = 5;
 
 // Graph-capture prefill: the arguments of a prefill launch and of its merge,
 // planned on the device (prefill.hip: prefill_capture_plan_kernel) from the

@@ -12,12 +12,20 @@ hipError_t launch_norm_rope(const NormRopeArgs &a, hipStream_t stream);
 // fp32: float inputs and output, else bf16; vec: 16-byte aligned rows and input.
 hipError_t launch_gemv(const GemvArgs &a, bool fp32, bool vec, hipStream_t stream);
 
-// Keys of one decode round for padded head dim `dp` and `qr` query vectors per
-// KV head (a power of two <= 8); an item of `rounds` rounds (1 or
-// kDecodeItemRounds) takes rounds times as many.
+// Rows with at most this many query vectors per KV head take a decode kernel,
+// with fp32 softmax weights up to kExactVectors of them.
+constexpr int kStreamMaxVectors = 32;
+constexpr int kExactVectors = 8;
+// 16-column groups of the decode kernel for a row of `vectors` query vectors
+// per KV head: up to 8 take three columns each (decode.hip: exact weights).
+constexpr int decode_column_groups(int vectors) {
+  return 3 * vectors <= 16 || (vectors > kExactVectors && vectors <= 16) ? 1 : 2;
+}
+// Keys one pass of a decode block's four waves takes for padded head dim `dp`.
 constexpr int kDecodeItemRounds = 4;
-int decode_tokens_per_item(int dp, int qr);
-hipError_t launch_decode(const AttnArgs &a, int dp, int qr, int rounds, int items, hipStream_t stream);
+int decode_tokens_per_item(int dp);
+constexpr int kDecodeWaves = 4;
+hipError_t launch_decode(const AttnArgs &a, int dp, int columns, int items, hipStream_t stream);
 
 hipError_t launch_prefill(const AttnArgs &a, int dp, hipStream_t stream);
 // The head-dim-256 prefill kernel over `blocks` blocks (prefill_d256.hip).
@@ -45,10 +53,9 @@ constexpr int kMergeSerialSplits = 8;
 hipError_t probe_xcd_dispatch(bool *round_robin, hipStream_t stream);
 
 // Graph-capture decode: the decode kernel over `blocks` blocks, then the merge
-// of every query vector of the capacity layout; max_splits = splits of a
-// row at capacity picks the merge's thread layout.
-hipError_t launch_decode_capture(const CaptureArgs &c, int dp, int qr, int rounds, int blocks, hipStream_t stream);
-hipError_t launch_merge_capture(const CaptureArgs &c, int dp, int max_splits, hipStream_t stream);
+// of every query vector of the capacity layout.
+hipError_t launch_decode_capture(const CaptureArgs &c, int dp, int columns, int blocks, hipStream_t stream);
+hipError_t launch_merge_capture(const CaptureArgs &c, int dp, hipStream_t stream);
 
 // Bytes of the static device scratch behind the allocation-free entry point
 // (XINFER_NOALLOC_SCRATCH_BYTES of the C header).

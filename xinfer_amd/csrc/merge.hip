@@ -27,31 +27,14 @@
 // gives its items, so the records a head's tiles wrote through one XCD's L2
 // are mostly read back on that XCD, and a vector's slices share the (m, l)
 // reads in one L2.
-#include "device_common.h"
 #include "kernel_args.h"
 #include "launch.h"
+#include "merge_common.h"
 
 namespace xattn {
 
 // Query vectors per prefill record block (the prefill kernel's query tile).
 constexpr int kMergeTile = 128;
-
-struct MergeState {
-  float m, l;
-  f32x4 o;
-};
-
-__device__ __forceinline__ void fold(MergeState &st, float ms, float ls, f32x4 os) {
-  if (ms == -INFINITY) return;
-  const float mn = fmaxf(st.m, ms);
-  const float a = fast_exp2(st.m - mn), w = fast_exp2(ms - mn);  // st.m = -inf -> a = 0
-  st.l = st.l * a + ls * w;
-  st.o.x = st.o.x * a + os.x * w;
-  st.o.y = st.o.y * a + os.y * w;
-  st.o.z = st.o.z * a + os.z * w;
-  st.o.w = st.o.w * a + os.w * w;
-  st.m = mn;
-}
 
 // LDS states of a block with SG > 1 split lanes over FS feature lanes.
 template <int FS, int SG>
@@ -237,24 +220,22 @@ static hipError_t launch_merge_d(const MergeArgs &a, const MergeArgs *dev, int m
 }
 
 // Graph-capture merge: one block per query vector of the capacity layout
-// (row, kv head, vector j < T * G), with split lanes over the splits.  The
-// row's count and length come from the device offsets; vectors past the row's
-// queries and rows whose keys fit one item (written by the decode kernel
+// (row, kv head, vector j < T * G), with split lanes over the splits.  Vectors
+// past the row's queries and rows of one split (written by the decode kernel
 // directly) have nothing to merge.
-template <int DP, int SG, int THREADS>
-__global__ void __launch_bounds__(THREADS) merge_capture_kernel(const CaptureArgs c) {
-  constexpr int FC = DP / 4;
-  static_assert(THREADS == FC * SG, "one query vector per block");
+template <int DP>
+__global__ void __launch_bounds__(256) merge_capture_kernel(const CaptureArgs c) {
+  constexpr int FC = DP / 4, SG = 256 / FC;
   __shared__ MergeRed<FC, SG> red;
-  const int tid = threadIdx.x, f = tid % FC, sg = tid / FC;
+  const int tid = threadIdx.x, lane = tid & 63, f = tid % FC, sg = tid / FC;
+  int count = 0, length = 1;
+  if (lane < c.B) capture_row(c, lane, count, length);
+  const int splits = capture_splits(c, lane, count, length);
   const int per_row = c.Hkv * c.T * c.G;
   const int r = (int)blockIdx.x / per_row, local = (int)blockIdx.x - r * per_row;
   const int qv_max = c.T * c.G;
   const int h = local / qv_max, j = local - h * qv_max;
-  int count, length;
-  capture_row(c, r, count, length);
-  const int qrows = count * c.G;
-  const int nsplit = (length + c.tok_item - 1) / c.tok_item;
+  const int qrows = __builtin_amdgcn_readlane(count, r) * c.G, nsplit = __builtin_amdgcn_readlane(splits, r);
   if (j >= qrows || nsplit <= 1) return;  // block-uniform
   const int d = f * 4;
   const int64_t ml_base = (int64_t)r * c.row_records + (int64_t)h * nsplit * qrows + j;
@@ -264,25 +245,14 @@ __global__ void __launch_bounds__(THREADS) merge_capture_kernel(const CaptureArg
                          d < c.D, sg, f, c.out + r * c.o_sb + (int64_t)(h * c.G + g) * c.o_sh + (int64_t)i * c.o_st + d);
 }
 
-template <int DP>
-static hipError_t launch_merge_capture_d(const CaptureArgs &c, int max_splits, hipStream_t stream) {
-  constexpr int FC = DP / 4;
-  const dim3 grid(c.total_items);
-  if (max_splits <= 16 * (256 / FC))
-    hipLaunchKernelGGL((merge_capture_kernel<DP, 256 / FC, 256>), grid, dim3(256), 0, stream, c);
-  else if (max_splits <= 16 * (512 / FC))
-    hipLaunchKernelGGL((merge_capture_kernel<DP, 512 / FC, 512>), grid, dim3(512), 0, stream, c);
-  else
-    hipLaunchKernelGGL((merge_capture_kernel<DP, 1024 / FC, 1024>), grid, dim3(1024), 0, stream, c);
-  return hipGetLastError();
-}
-
-hipError_t launch_merge_capture(const CaptureArgs &c, int dp, int max_splits, hipStream_t stream) {
+hipError_t launch_merge_capture(const CaptureArgs &c, int dp, hipStream_t stream) {
+  const dim3 grid(c.B * c.Hkv * c.T * c.G);
   switch (dp) {
-    case 64: return launch_merge_capture_d<64>(c, max_splits, stream);
-    case 128: return launch_merge_capture_d<128>(c, max_splits, stream);
-    default: return launch_merge_capture_d<256>(c, max_splits, stream);
+    case 64: hipLaunchKernelGGL(merge_capture_kernel<64>, grid, dim3(256), 0, stream, c); break;
+    case 128: hipLaunchKernelGGL(merge_capture_kernel<128>, grid, dim3(256), 0, stream, c); break;
+    default: hipLaunchKernelGGL(merge_capture_kernel<256>, grid, dim3(256), 0, stream, c); break;
   }
+  return hipGetLastError();
 }
 
 hipError_t launch_merge(const MergeArgs &a, int dp, int max_splits, hipStream_t stream) {
