@@ -20,119 +20,155 @@
 // a sum whose order differs between implementations, may differ in its last
 // bit.
 //
-// One row = (token, projected head): the Hq query heads, then the Hkv key
+// A row is a (token, projected head): the Hq query heads, then the Hkv key
 // heads, then the Hkv value heads of each token.  LPR = D/8 lanes hold a row,
-// 8 features (16 bytes) each; a 256-thread block holds 256/LPR rows.  The
-// partner of lane c for the rotation is lane c ^ LPR/2 (the other half of the
-// row).  A key or value row is written to the cache only for a real token
-// (t < count_r) whose position lies in [0, C); query rows are written for
-// every token, as the eager sequence computes them.
+// 8 features (16 bytes) each; a block takes one token, and its waves in turn
+// take 64/LPR heads of one kind at a time (a task).  The partner of lane c for
+// the rotation is lane c ^ LPR/2 (the other half of the row).  A key or value row
+// is written to the cache only for a real token (t < count_r) whose position lies
+// in [0, C); query rows are written for every token, as the eager sequence
+// computes them.
+//
+// What bounds it: latency for a few tokens; for many the vector arithmetic and
+// the waves' start (a row is 256 bytes at D = 128, and its rounding points take
+// some 120 instructions).  So a task's kind, its addresses and its token's count
+// and position are scalar work without a division, value rows are copied,
+// roundings and the partner's exchange go two features at a time, and with many
+// tokens the key and value rows of padded ones are not read.  Against one row per
+// lane group with all of that per lane (16 query and 8 KV heads, D = 128, in
+// graph replays): 8 x 384 tokens of which 391 are real 17.1 -> 11.1 us, 8 x 512
+// real ones 22.0 -> 17.7 us (4.3 TB/s), 512 tokens 5.2 us both, 8 tokens
+// 3.16 -> 3.10 us.
+#include <algorithm>
+
 #include "device_common.h"
 #include "kernel_args.h"
 
 namespace xattn {
 
-__device__ __forceinline__ float round_bf16(float x) { return __uint_as_float(f32_to_bf16_bits(x) << 16); }
+// Two floats rounded to bf16: a packed pair of bits.
+__device__ __forceinline__ uint32_t round2(float lo, float hi) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
+}
+
+// The partner lane's word (the other half of the row): DPP row_ror:8 within a
+// 16-lane row (LPR = 16), the permlane16 swap (LPR = 32); a shuffle through LDS
+// for LPR = 8.
+template <int LPR>
+__device__ __forceinline__ uint32_t partner_word(uint32_t x, int dc) {
+  if constexpr (LPR == 16) {
+    return __float_as_uint(dpp_move<kDppRowRor8>(__uint_as_float(x)));
+  } else if constexpr (LPR == 32) {
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    return dc < 16 ? r[1] : r[0];
+  } else {
+    return (uint32_t)__shfl_xor((int)x, LPR / 2, LPR);
+  }
+}
+
+// Eight floats of a packed bf16 chunk.
+struct Floats8 {
+  float f[8];
+};
+__device__ __forceinline__ Floats8 unpack8(const u32x4 &x) {
+  Floats8 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    r.f[2 * e] = bf16_lo(x[e]);
+    r.f[2 * e + 1] = bf16_hi(x[e]);
+  }
+  return r;
+}
+
+// The normalised and rotated row (x: 8 features of it, w the norm weights, cs and
+// sn the rotary tables).  The LPR lanes of a row call it together.
+template <int LPR>
+__device__ __forceinline__ u32x4 norm_rope(const u32x4 &x, const Floats8 &w, const Floats8 &cs, const Floats8 &sn,
+                                           float eps, int dc) {
+  const Floats8 xf = unpack8(x);
+  float ss = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ss = fmaf(xf.f[e], xf.f[e], ss);  // x^2 is exact in fp32
+  ss = group_sum<LPR>(ss);
+  const float inv = rsqrtf(ss / (float)(LPR * 8) + eps);
+  // The rotation's sign: rot = -partner in the lower half of the row.
+  const uint32_t sign = dc < LPR / 2 ? 0x80008000u : 0u;
+  u32x4 out;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t y = round2(xf.f[2 * e] * inv, xf.f[2 * e + 1] * inv);
+    const uint32_t xn = round2(w.f[2 * e] * bf16_lo(y), w.f[2 * e + 1] * bf16_hi(y));
+    const uint32_t rot = partner_word<LPR>(xn, dc) ^ sign;
+    const uint32_t p = round2(bf16_lo(xn) * cs.f[2 * e], bf16_hi(xn) * cs.f[2 * e + 1]);
+    const uint32_t q = round2(bf16_lo(rot) * sn.f[2 * e], bf16_hi(rot) * sn.f[2 * e + 1]);
+    out[e] = round2(bf16_lo(p) + bf16_lo(q), bf16_hi(p) + bf16_hi(q));
+  }
+  return out;
+}
+
+// Tokens from which blocks have 4 waves, which take several tasks each, and skip
+// padded keys and values.  Below, 8 waves start all loads at once, before the
+// position arrives.  (8 against 4 waves: 512 tokens 5.5 / 5.8 us, 1024 tokens at
+// D = 256 10.6 / 11.5; 2048 tokens 12.3 / 11.2, 8 x 384 14.5 / 11.6, 2048 tokens at
+// D = 256 16.6 / 15.8.)
+constexpr int64_t kNormRopeManyTokens = 2048;
+constexpr int kNormRopeGridRows = 65535;
+constexpr int norm_rope_threads(bool many) { return many ? 256 : 512; }
+
+template <int LPR, bool MANY>
+__global__ void __launch_bounds__(norm_rope_threads(MANY), MANY ? 4 : 2) norm_rope_kernel(const NormRopeArgs a) {
+  constexpr int HEADS = 64 / LPR;  // heads of a task
+  const int lane = threadIdx.x & 63, head = lane / LPR, dc = lane % LPR;
+  const int b = (int)(blockIdx.z * kNormRopeGridRows + blockIdx.y), t = (int)blockIdx.x;
+  if (b >= a.B) return;
+  // The row's count and the token's position are block-uniform scalar loads.
+  typedef const __attribute__((address_space(4))) int32_t *counts_ptr;
+  typedef const __attribute__((address_space(4))) int64_t *positions_ptr;
+  const counts_ptr cu = (counts_ptr)a.cu_query;
+  const int64_t pos = ((positions_ptr)a.positions)[b * a.pos_sb + t * a.pos_st];
+  const int count = cu[b + 1] - cu[b];
+  const int q_tasks = (a.Hq + HEADS - 1) / HEADS, kv_tasks = (a.Hkv + HEADS - 1) / HEADS;
+  for (int task = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); task < q_tasks + 2 * kv_tasks;
+       task += norm_rope_threads(MANY) / 64) {
+    const bool query = task < q_tasks, value = task >= q_tasks + kv_tasks;
+    const int h = (task - (query ? 0 : (value ? q_tasks + kv_tasks : q_tasks))) * HEADS + head;
+    const int heads = query ? a.Hq : a.Hkv;
+    const bool real = t < count && pos >= 0 && pos < a.C;
+    if (MANY && !query && !real) break;
+    const View &src = query ? a.q : (value ? a.v : a.k);
+    // Lanes past the last head repeat it; they write nothing.
+    u32x4 out = load16(src.p + b * src.sb + t * src.st + (int64_t)min(h, heads - 1) * src.sh + dc * 8);
+    if (!value) {
+      const u32x4 w = load16((query ? a.q_weight : a.k_weight) + dc * 8);
+      const u32x4 cs = load16(a.cos.p + b * a.cos.sb + t * a.cos.st + dc * 8);
+      const u32x4 sn = load16(a.sin.p + b * a.sin.sb + t * a.sin.st + dc * 8);
+      out = norm_rope<LPR>(out, unpack8(w), unpack8(cs), unpack8(sn), a.eps, dc);
+    }
+    if (query) {
+      if (h < heads) store16(a.q_out + (((int64_t)b * a.Hq + h) * a.T + t) * (LPR * 8) + dc * 8, out);
+    } else if (real && h < heads) {
+      store16((value ? a.cache_value : a.cache_key) + (((int64_t)b * a.Hkv + h) * a.C + pos) * (LPR * 8) + dc * 8, out);
+    }
+  }
+}
 
 template <int LPR>
-__global__ void __launch_bounds__(256) norm_rope_kernel(const NormRopeArgs a) {
-  constexpr int ROWS = 256 / LPR;
-  const int lane_row = threadIdx.x / LPR, dc = threadIdx.x % LPR;
-  const int64_t grow = (int64_t)blockIdx.x * ROWS + lane_row;
-  const int per_token = a.Hq + 2 * a.Hkv;
-  const int64_t token = grow / per_token;
-  if (token >= (int64_t)a.B * a.T) return;  // whole rows only: LPR lanes exit together
-  const int which = (int)(grow - token * per_token);
-  const int b = (int)(token / a.T), t = (int)(token - (int64_t)b * a.T);
-  const int kind = which < a.Hq ? 0 : (which < a.Hq + a.Hkv ? 1 : 2);  // query, key, value
-  const int h = kind == 0 ? which : (kind == 1 ? which - a.Hq : which - a.Hq - a.Hkv);
-  const View &src = kind == 0 ? a.q : (kind == 1 ? a.k : a.v);
-
-  // Every load of the row in one round trip.
-  const u32x4 x = load16(src.p + b * src.sb + h * src.sh + t * src.st + dc * 8);
-  u32x4 w{0, 0, 0, 0}, cs{0, 0, 0, 0}, sn{0, 0, 0, 0};
-  if (kind < 2) {
-    w = load16((kind == 0 ? a.q_weight : a.k_weight) + dc * 8);
-    cs = load16(a.cos.p + b * a.cos.sb + t * a.cos.st + dc * 8);
-    sn = load16(a.sin.p + b * a.sin.sb + t * a.sin.st + dc * 8);
-  }
-  int32_t c0 = 0, c1 = 0;
-  int64_t pos = -1;
-  if (kind > 0) {
-    c0 = as_global(a.cu_query)[b];
-    c1 = as_global(a.cu_query)[b + 1];
-    pos = as_global(a.positions)[b * a.pos_sb + t * a.pos_st];
-  }
-
-  u32x4 outw = x;
-  if (kind < 2) {
-    float xf[8];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      xf[2 * e] = bf16_lo(x[e]);
-      xf[2 * e + 1] = bf16_hi(x[e]);
-    }
-    float ss = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ss = fmaf(xf[e], xf[e], ss);  // x^2 is exact in fp32
-    ss = group_sum<LPR>(ss);
-    const float inv = rsqrtf(ss / (float)(LPR * 8) + a.eps);
-    float xn[8];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      xn[2 * e] = round_bf16(bf16_lo(w[e]) * round_bf16(xf[2 * e] * inv));
-      xn[2 * e + 1] = round_bf16(bf16_hi(w[e]) * round_bf16(xf[2 * e + 1] * inv));
-    }
-    // The other half of the row, from the partner lane c ^ LPR/2: DPP
-    // row_ror:8 within a 16-lane row (LPR = 16), the permlane16 swap (LPR =
-    // 32); a shuffle through LDS for LPR = 8.
-    float pn[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      if constexpr (LPR == 16) {
-        pn[e] = dpp_move<kDppRowRor8>(xn[e]);
-      } else if constexpr (LPR == 32) {
-        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(xn[e]), __float_as_uint(xn[e]), false, false);
-        pn[e] = __uint_as_float(dc < 16 ? r[1] : r[0]);
-      } else {
-        pn[e] = __shfl_xor(xn[e], LPR / 2, LPR);
-      }
-    }
-    const bool lower = dc < LPR / 2;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float o[2];
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int i = 2 * e + u;
-        const float c = u ? bf16_hi(cs[e]) : bf16_lo(cs[e]);
-        const float s = u ? bf16_hi(sn[e]) : bf16_lo(sn[e]);
-        const float rot = lower ? -pn[i] : pn[i];
-        o[u] = round_bf16(round_bf16(xn[i] * c) + round_bf16(rot * s));
-      }
-      outw[e] = pack_bf16x2(o[0], o[1]);
-    }
-  }
-
-  if (kind == 0) {
-    store16(a.q_out + ((int64_t)(b * a.Hq + h) * a.T + t) * (LPR * 8) + dc * 8, outw);
-    return;
-  }
-  int count = c1 - c0;
-  count = count < 0 ? 0 : (count > a.T ? a.T : count);
-  if (t >= count || pos < 0 || pos >= a.C) return;
-  uint16_t *cache = kind == 1 ? a.cache_key : a.cache_value;
-  store16(cache + (((int64_t)b * a.Hkv + h) * a.C + pos) * (LPR * 8) + dc * 8, outw);
+static void launch_norm_rope_d(const NormRopeArgs &a, hipStream_t stream) {
+  const int64_t tokens = (int64_t)a.B * a.T;
+  const bool many = tokens >= kNormRopeManyTokens;
+  // Tokens by rows (no division in the kernel); a grid takes 65535 rows in y.
+  const dim3 grid(a.T, std::min(a.B, kNormRopeGridRows), (a.B + kNormRopeGridRows - 1) / kNormRopeGridRows);
+  const dim3 block(norm_rope_threads(many));
+  if (many) hipLaunchKernelGGL((norm_rope_kernel<LPR, true>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((norm_rope_kernel<LPR, false>), grid, block, 0, stream, a);
 }
 
 hipError_t launch_norm_rope(const NormRopeArgs &a, hipStream_t stream) {
-  const int64_t rows = (int64_t)a.B * a.T * (a.Hq + 2 * a.Hkv);
-  const int lpr = a.D / 8;
-  const dim3 grid((unsigned)((rows * lpr + 255) / 256));
-  switch (lpr) {
-    case 8: hipLaunchKernelGGL((norm_rope_kernel<8>), grid, dim3(256), 0, stream, a); break;
-    case 16: hipLaunchKernelGGL((norm_rope_kernel<16>), grid, dim3(256), 0, stream, a); break;
-    default: hipLaunchKernelGGL((norm_rope_kernel<32>), grid, dim3(256), 0, stream, a); break;
+  switch (a.D) {
+    case 64: launch_norm_rope_d<8>(a, stream); break;
+    case 128: launch_norm_rope_d<16>(a, stream); break;
+    default: launch_norm_rope_d<32>(a, stream); break;
   }
   return hipGetLastError();
 }
