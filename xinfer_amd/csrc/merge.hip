@@ -130,7 +130,7 @@ __device__ __forceinline__ void merge_body(const MergeArgs &a) {
   const int vec = SG > 1 ? group / NS : group * VPB + vl;
   const int f = SG > 1 ? (group - vec * NS) * FS + fl : fl;  // feature lane of the vector
   const bool vvalid = vec < total_items;
-  const MergeRow mr = rows.find(a.rows, nrows, vvalid ? vec : 0);
+  const MergeRow mr = rows.template find<(SG > 1)>(a.rows, nrows, vvalid ? vec : 0);
   const int local = vec - mr.item_begin;
   const int qrows = mr.count * G;
   const int h = local / qrows, j = local - h * qrows;
