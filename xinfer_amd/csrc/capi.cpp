@@ -181,13 +181,22 @@ DecodeChoice choose_decode(const Geometry &g, const std::vector<int32_t> &counts
   if (items[0] >= kDecodeManyItems || widest > kExactVectors || prefill) {
     // The fewest passes per item that leave at most `limit` items.
     auto least = [&](int64_t limit) {
-      int64_t m = std::max<int64_t>(1, ceil_div(items[0], limit));
-      for (; m < longest; ++m) {
+      auto fits = [&](int64_t m) {  // items only fall as m grows
         int64_t count = 0;
-        for (int r = 0; r < n; ++r) count += g.Hkv * ceil_div(passes[r], m);
-        if (count <= std::max(limit, pairs)) break;
+        for (int r = 0; r < n; ++r) count += ((uint32_t)passes[r] + (uint32_t)m - 1) / (uint32_t)m;
+        return g.Hkv * count <= std::max(limit, pairs);
+      };
+      int64_t low = std::max<int64_t>(1, ceil_div(items[0], limit)), high = low;
+      for (int64_t step = 1; high < longest && !fits(high); step *= 2) {
+        low = high + 1;
+        high = std::min(longest, high + step);
       }
-      return m;
+      while (low < high) {
+        const int64_t m = (low + high) / 2;
+        if (fits(m)) high = m;
+        else low = m + 1;
+      }
+      return low;
     };
     auto even = [&](int64_t m, int64_t limit) { return m * limit * kDecodeEvenDen <= items[0] * kDecodeEvenNum; };
     const int64_t m1 = least(kDecodeCus), m2 = least(2 * kDecodeCus);
