@@ -41,7 +41,7 @@ struct DecodeItem {
   int b, h, split, nsplit, cnt, L, t0, t1;
   int kvb;      // cache row of the item's K/V: b, or b's page
   int counter;  // arrival counter of this (row, kv head)
-  int64_t rec_begin;
+  int64_t rec;  // first record of the item (its splits' records follow one another)
 };
 
 // The arguments a decode block uses (named as in AttnArgs), pinned in SGPRs by
@@ -57,9 +57,9 @@ struct DecodeParams {
   uint64_t tag;
 };
 
-// per: keys of one split.
+// per: keys of one split; rec: the item's first record.
 __device__ __forceinline__ DecodeItem make_item(int batch, int count, int length, int nsplit, int per, int h,
-                                                int split, int counter, int64_t rec_begin) {
+                                                int split, int counter, int64_t rec) {
   DecodeItem it;
   it.h = h;
   it.split = split;
@@ -71,7 +71,7 @@ __device__ __forceinline__ DecodeItem make_item(int batch, int count, int length
   it.t0 = split * per;
   it.t1 = min(length, it.t0 + per);
   it.counter = counter;
-  it.rec_begin = rec_begin;
+  it.rec = rec;
   return it;
 }
 
@@ -153,7 +153,7 @@ __device__ void merge_in_launch(const DecodeParams &a, const DecodeItem &it, int
   constexpr int FQ = DP / 4;  // feature quads of a padded vector
   const int D = a.D, G = a.G, nsplit = it.nsplit;
   // Record (split s, vector j) of this (row, kv head): rec0 + s * qrows + j.
-  const int64_t rec0 = it.rec_begin + (int64_t)it.h * nsplit * qrows;
+  const int64_t rec0 = it.rec - (int64_t)it.split * qrows;
   const __amdgpu_buffer_rsrc_t o_rsrc = buffer_rsrc(a.part_o + rec0 * D, (uint32_t)(nsplit * qrows * D * 4));
   const __amdgpu_buffer_rsrc_t ml_rsrc = buffer_rsrc(a.part_ml + 2 * rec0, (uint32_t)(nsplit * qrows * 8));
   for (int idx = tid; idx < qrows * FQ; idx += kItemThreads) {
@@ -259,7 +259,7 @@ __device__ __forceinline__ void process_item(const DecodeParams &a, DecodeItem &
           *as_global(reinterpret_cast<u32x2 *>(dst)) =
               u32x2{pack_bf16x2(o[0] / l, o[1] / l), pack_bf16x2(o[2] / l, o[3] / l)};
         } else {
-          const int64_t rec = it.rec_begin + ((int64_t)it.h * it.nsplit + it.split) * qrows + j;
+          const int64_t rec = it.rec + j;
           *as_global(reinterpret_cast<f32x4 *>(a.part_o + rec * D + d)) = o;
           if (d == 0)
             *as_global(reinterpret_cast<u32x2 *>(a.part_ml + 2 * rec)) =
@@ -291,7 +291,8 @@ __global__ void __launch_bounds__(kItemThreads, 2) decode_kernel(const AttnArgs 
     const int item = blockIdx.x;
     const RowSched rs = rows.find(a.rows, nrows, item);
     const int local = item - rs.item_begin, h = local / rs.nsplit;
-    it = make_item(rs.batch, rs.count, rs.length, rs.nsplit, rs.ntiles, h, local - h * rs.nsplit, 0, rs.rec_begin);
+    it = make_item(rs.batch, rs.count, rs.length, rs.nsplit, rs.ntiles, h, local - h * rs.nsplit, 0,
+                   rs.rec_begin + (int64_t)local * (rs.count * p.G));
   } else {
     // In-launch merge (Hkv a multiple of 8): block b runs on XCD x = b % 8 and
     // takes, row after row, the items of the kv heads h = x (mod 8), so every
@@ -302,8 +303,9 @@ __global__ void __launch_bounds__(kItemThreads, 2) decode_kernel(const AttnArgs 
     const RowSched rs = rows.find(a.rows, nrows, 8 * slot);
     const int local = slot - rs.item_begin / 8, hh = local / rs.nsplit;
     const int h = 8 * hh + x;
-    it = make_item(rs.batch, rs.count, rs.length, rs.nsplit, rs.ntiles, h, local - hh * rs.nsplit,
-                   rs.item_begin + h * rs.nsplit, rs.rec_begin);
+    const int split = local - hh * rs.nsplit;
+    it = make_item(rs.batch, rs.count, rs.length, rs.nsplit, rs.ntiles, h, split, rs.item_begin + h * rs.nsplit,
+                   rs.rec_begin + (int64_t)(h * rs.nsplit + split) * (rs.count * p.G));
   }
   // The page is read while the loads issued for row it.b are in flight.
   const int raw_page = read_page(blocks, blocks_stride, it.b);
@@ -329,10 +331,10 @@ __global__ void __launch_bounds__(kItemThreads, 2) decode_capture_kernel(const C
   const int r = __popcll(before) - 1;  // row 0 begins at 0
   if (item >= __builtin_amdgcn_readlane(end, r)) return;
   const int row_splits = __builtin_amdgcn_readlane(nsplit, r), local = item - __builtin_amdgcn_readlane(begin, r);
-  const int h = local / row_splits;
+  const int h = local / row_splits, split = local - h * row_splits;
   DecodeItem it = make_item(r, __builtin_amdgcn_readlane(count, r), __builtin_amdgcn_readlane(length, r), row_splits,
-                            __builtin_amdgcn_readlane(per, r), h, local - h * row_splits, 0,
-                            (int64_t)r * c.row_records);
+                            __builtin_amdgcn_readlane(per, r), h, split, 0,
+                            r * c.row_records + (int64_t)(h * c.splits_max + split) * (c.T * c.G));
   const DecodeParams p{c.q, c.k, c.v, c.out, c.o_sb, c.o_sh, c.o_st, c.part_o, c.part_ml, c.scale_log2, c.D, c.G, c.T};
   process_item<DP, NC>(p, it, read_page(c.blocks, c.blocks_stride, r), c.B, smem);
 }

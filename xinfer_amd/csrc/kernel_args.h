@@ -94,8 +94,8 @@ struct CaptureArgs {
   int32_t D, G, Hkv, T, B, C;
   const int32_t *blocks;     // page table as in AttnArgs (nullable), over the B rows of k/v
   int64_t blocks_stride;
-  // Decode: row r's records start at r * row_records, [kv head][split][vector]
-  // with the row's splits (device_common.h: capture_splits).
+  // Decode: row r's records start at r * row_records, [kv head][splits_max][T * G],
+  // of which the row's splits (device_common.h: capture_splits) and vectors are used.
   int64_t row_records;
   int32_t pass_keys;         // keys a block's waves take together
   int32_t pass_min;          // least passes per item

@@ -40,9 +40,11 @@ constexpr int kMergeTile = 128;
 template <int FS, int SG>
 using MergeRed = MergeState[SG > 1 ? SG : 1][SG > 1 ? FS : 1];
 
-// Folds the nsplit records of one query vector over this thread's 4 features
-// and writes them as bf16 at dst.  Record s: o at part_o + o_base + s * o_step,
-// (m, l) at part_ml + 2 * (ml_base + s * ml_step).  With SG > 1 split lanes
+constexpr MergeState kMergeStart{-INFINITY, 0.0f, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+
+// Folds records first, first + SG, ... below nsplit of one query vector into st over
+// this thread's 4 features and writes them as bf16 at dst.  Record s: o at
+// part_o + o_base + s * o_step, (m, l) at part_ml + 2 * (ml_base + s * ml_step).  With SG > 1 split lanes
 // per feature group every thread of the block must call it (it synchronises
 // the block); `active` is false for threads past the vectors or features, and
 // f is the thread's feature lane within the block's FS.  Every record of a
@@ -51,11 +53,11 @@ using MergeRed = MergeState[SG > 1 ? SG : 1][SG > 1 ? FS : 1];
 template <int FS, int SG>
 __device__ __forceinline__ void fold_and_write(MergeRed<FS, SG> &red, const float *part_o, const float *part_ml,
                                                int64_t o_base, int64_t o_step, int64_t ml_base, int64_t ml_step,
-                                               int nsplit, bool active, int sg, int f, uint16_t *dst) {
+                                               int nsplit, bool active, int sg, int f, uint16_t *dst, MergeState st,
+                                               int first) {
   constexpr int INFLIGHT = SG > 1 ? 16 : 4;
-  MergeState st{-INFINITY, 0.0f, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
   if (active) {
-    for (int s0 = sg; s0 < nsplit; s0 += INFLIGHT * SG) {
+    for (int s0 = first; s0 < nsplit; s0 += INFLIGHT * SG) {
       u32x2 ml[INFLIGHT];
       f32x4 o[INFLIGHT];
 #pragma unroll
@@ -154,7 +156,7 @@ __device__ __forceinline__ void merge_body(const MergeArgs &a) {
 
   const int g = j % G, i = j / G;
   fold_and_write<FS, SG>(red, part_o, part_ml, o_base, o_step, ml_base, ml_step, mr.nsplit, vvalid && d < D, sg, fl,
-                         out + mr.batch * o_sb + (int64_t)(h * G + g) * o_sh + (int64_t)i * o_st + d);
+                         out + mr.batch * o_sb + (int64_t)(h * G + g) * o_sh + (int64_t)i * o_st + d, kMergeStart, sg);
 }
 
 // Feature lanes per block past kMergeSliceSplits splits: 64 features, 256
@@ -222,27 +224,51 @@ static hipError_t launch_merge_d(const MergeArgs &a, const MergeArgs *dev, int m
 // Graph-capture merge: one block per query vector of the capacity layout
 // (row, kv head, vector j < T * G), with split lanes over the splits.  Vectors
 // past the row's queries and rows of one split (written by the decode kernel
-// directly) have nothing to merge.
+// directly) have nothing to merge.  A block waits for the device's lengths before
+// it knows its splits; the records' places do not depend on them, so in small
+// launches a lane's first records are loaded beside the lengths, whether its row
+// has them or not (the workspace holds them all): eight layers' captured steps of
+// 8 rows, 128 vectors, 156.4 -> 150.3 us.  Larger launches, whose records past the
+// splits would be a load worth saving (2 KB a split lane; 512 vectors: 8 MB at
+// most), wait.
+constexpr int kMergeAheadVectors = 512;
+
 template <int DP>
 __global__ void __launch_bounds__(256) merge_capture_kernel(const CaptureArgs c) {
-  constexpr int FC = DP / 4, SG = 256 / FC;
+  constexpr int FC = DP / 4, SG = 256 / FC, AHEAD = 4;
   __shared__ MergeRed<FC, SG> red;
-  const int tid = threadIdx.x, lane = tid & 63, f = tid % FC, sg = tid / FC;
+  const int tid = threadIdx.x, lane = tid & 63, f = tid % FC, sg = tid / FC, d = f * 4;
+  const int qv_max = c.T * c.G, per_row = c.Hkv * qv_max;
+  const int r = (int)blockIdx.x / per_row, local = (int)blockIdx.x - r * per_row;
+  const int h = local / qv_max, j = local - h * qv_max;
+  const int64_t ml_base = r * c.row_records + (int64_t)h * c.splits_max * qv_max + j, ml_step = qv_max;
+  const int64_t o_base = ml_base * c.D + d, o_step = ml_step * c.D;
+  const bool ahead = gridDim.x <= kMergeAheadVectors;
+  u32x2 ml[AHEAD];
+  f32x4 o[AHEAD];
+  if (ahead && d < c.D) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (sg + u * SG < c.splits_max) {
+        ml[u] = *as_global(reinterpret_cast<const u32x2 *>(c.part_ml + 2 * (ml_base + (sg + u * SG) * ml_step)));
+        o[u] = *as_global(reinterpret_cast<const f32x4 *>(c.part_o + o_base + (sg + u * SG) * o_step));
+      }
+  }
   int count = 0, length = 1;
   if (lane < c.B) capture_row(c, lane, count, length);
   const int splits = capture_splits(c, lane, count, length);
-  const int per_row = c.Hkv * c.T * c.G;
-  const int r = (int)blockIdx.x / per_row, local = (int)blockIdx.x - r * per_row;
-  const int qv_max = c.T * c.G;
-  const int h = local / qv_max, j = local - h * qv_max;
   const int qrows = __builtin_amdgcn_readlane(count, r) * c.G, nsplit = __builtin_amdgcn_readlane(splits, r);
   if (j >= qrows || nsplit <= 1) return;  // block-uniform
-  const int d = f * 4;
-  const int64_t ml_base = (int64_t)r * c.row_records + (int64_t)h * nsplit * qrows + j;
-  const int64_t ml_step = qrows;
+  MergeState st = kMergeStart;
+  if (ahead && d < c.D) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (sg + u * SG < nsplit) fold(st, __uint_as_float(ml[u].x), __uint_as_float(ml[u].y), o[u]);
+  }
   const int g = j % c.G, i = j / c.G;
-  fold_and_write<FC, SG>(red, c.part_o, c.part_ml, ml_base * c.D + d, ml_step * c.D, ml_base, ml_step, nsplit,
-                         d < c.D, sg, f, c.out + r * c.o_sb + (int64_t)(h * c.G + g) * c.o_sh + (int64_t)i * c.o_st + d);
+  fold_and_write<FC, SG>(red, c.part_o, c.part_ml, o_base, o_step, ml_base, ml_step, nsplit, d < c.D, sg, f,
+                         c.out + r * c.o_sb + (int64_t)(h * c.G + g) * c.o_sh + (int64_t)i * c.o_st + d, st,
+                         ahead ? sg + AHEAD * SG : sg);
 }
 
 hipError_t launch_merge_capture(const CaptureArgs &c, int dp, hipStream_t stream) {
