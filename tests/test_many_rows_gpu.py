@@ -17,18 +17,11 @@ from xinfer_amd.attention import batched_attention_metadata
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("rows", (9, 64, 67))
-@pytest.mark.parametrize("what", ("decode", "mixed", "prefill"))
-@pytest.mark.parametrize("dim", (64, 256))
-@torch.inference_mode()
-def test_every_row_of_a_launch(gpu_ops, rows, what, dim):
-    heads, kv_heads, capacity = (8, 8, 1501) if what == "decode" else (4, 1, 1501)
-    counts = [{"decode": 1, "mixed": (1, 40, 2)[r % 3], "prefill": 33 + r % 5}[what] for r in range(rows)]
-    lengths = [n + (r * 389 + (0 if r % 2 else 1100)) % (capacity - 40) for r, n in enumerate(counts)]
-    log(f"rows of a launch {what} rows={rows} D={dim} Hq={heads} Hkv={kv_heads}")
-    generator = torch.Generator().manual_seed(rows)
-    q = torch.randn(rows, heads, max(counts), dim, generator=generator).to(torch.bfloat16)
-    k, v = (torch.randn(rows, kv_heads, capacity, dim, generator=generator).to(torch.bfloat16) for _ in range(2))
+def check(gpu_ops, heads, kv_heads, dim, counts, lengths, capacity):
+    generator = torch.Generator().manual_seed(len(counts))
+    q = torch.randn(len(counts), heads, max(counts), dim, generator=generator).to(torch.bfloat16)
+    k, v = (torch.randn(len(counts), kv_heads, capacity, dim, generator=generator).to(torch.bfloat16)
+            for _ in range(2))
     host, cu, blocks = batched_attention_metadata(
         torch.tensor(lengths, dtype=torch.int32), torch.tensor(counts, dtype=torch.int32), "cuda")
     out = gpu_ops.batched_flash_attention(q.cuda(), k.cuda(), v.cuda(), host, cu, blocks, dim ** -0.5).cpu()
@@ -39,3 +32,24 @@ def test_every_row_of_a_launch(gpu_ops, rows, what, dim):
                             torch.from_numpy(expected[r:r + 1, :, :count]).float().flatten(1))
         assert errors["max_abs"] <= MAX_ABS and errors["mean_abs"] <= MEAN_ABS, (r, errors)
         assert errors["relative_l2"] < 0.01 and errors["peak_relative"] <= 0.05, (r, errors)
+
+
+@pytest.mark.parametrize("rows", (9, 64, 67))
+@pytest.mark.parametrize("what", ("decode", "mixed", "prefill"))
+@pytest.mark.parametrize("dim", (64, 256))
+@torch.inference_mode()
+def test_every_row_of_a_launch(gpu_ops, rows, what, dim):
+    heads, kv_heads, capacity = (8, 8, 1501) if what == "decode" else (4, 1, 1501)
+    counts = [{"decode": 1, "mixed": (1, 40, 2)[r % 3], "prefill": 33 + r % 5}[what] for r in range(rows)]
+    lengths = [n + (r * 389 + (0 if r % 2 else 1100)) % (capacity - 40) for r, n in enumerate(counts)]
+    log(f"rows of a launch {what} rows={rows} D={dim} Hq={heads} Hkv={kv_heads}")
+    check(gpu_ops, heads, kv_heads, dim, counts, lengths, capacity)
+
+
+@pytest.mark.parametrize("dim", (64, 72, 128, 256))
+@torch.inference_mode()
+def test_decode_and_prefill_rows_merge_together(gpu_ops, dim):
+    """Decode rows of more than eight splits (and of fewer) beside split prefill rows."""
+    counts, lengths = [1, 40, 2, 33, 1, 65], [3000, 2900, 2400, 1500, 700, 513]
+    log(f"merge of both kinds D={dim} counts={counts} lengths={lengths}")
+    check(gpu_ops, 12, 3, dim, counts, lengths, 3001)

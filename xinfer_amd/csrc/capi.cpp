@@ -637,21 +637,26 @@ int run_plan(const Plan &plan, const Geometry &g, const xinfer_view4 &q, const x
     if (grp.dec_items > 0 && launch_decode(grp.dec, dp, grp.dec_columns, grp.dec_items, stream) != hipSuccess)
       return XINFER_ERR_LAUNCH;
     if (grp.pre_items > 0 && launch_prefill(grp.pre, dp, stream) != hipSuccess) return XINFER_ERR_LAUNCH;
-    for (const bool decode : {true, false}) {
-      MergeArgs &m = decode ? grp.dec_merge : grp.pre_merge;
-      m.total_items = decode ? grp.dec_merge_items : grp.pre_merge_items;
-      if (m.total_items == 0) continue;
-      m.out = static_cast<uint16_t *>(const_cast<void *>(out.data));
-      m.o_sb = out.stride[0];
-      m.o_sh = out.stride[1];
-      m.o_st = out.stride[2];
-      m.part_o = part_o;
-      m.part_ml = part_ml;
-      m.D = (int32_t)g.D;
-      m.G = G;
-      if (launch_merge(m, dp, decode ? grp.dec_max_splits : grp.pre_max_splits, stream) != hipSuccess)
-        return XINFER_ERR_LAUNCH;
+    grp.dec_merge.total_items = grp.dec_merge_items;
+    grp.pre_merge.total_items = grp.pre_merge_items;
+    for (MergeArgs *m : {&grp.dec_merge, &grp.pre_merge}) {
+      m->out = static_cast<uint16_t *>(const_cast<void *>(out.data));
+      m->o_sb = out.stride[0];
+      m->o_sh = out.stride[1];
+      m->o_st = out.stride[2];
+      m->part_o = part_o;
+      m->part_ml = part_ml;
+      m->D = (int32_t)g.D;
+      m->G = G;
     }
+    hipError_t rc = hipSuccess;
+    if (grp.dec_merge_items > 0 && grp.pre_merge_items > 0)
+      rc = launch_merge_both(grp.dec_merge, grp.pre_merge, dp, grp.dec_max_splits, grp.pre_max_splits, stream);
+    else if (grp.dec_merge_items > 0)
+      rc = launch_merge(grp.dec_merge, dp, grp.dec_max_splits, stream);
+    else if (grp.pre_merge_items > 0)
+      rc = launch_merge(grp.pre_merge, dp, grp.pre_max_splits, stream);
+    if (rc != hipSuccess) return XINFER_ERR_LAUNCH;
   }
   return XINFER_OK;
 }

@@ -75,6 +75,7 @@ struct MergeArgs {
   const float *part_ml;
   int32_t D, G;
   int32_t total_items;  // query vectors to merge
+  int32_t lane_items;   // merge_both: the first of them have rows of many splits, the others few
   int32_t nrows;
   MergeRow rows[kMaxRows];
 };

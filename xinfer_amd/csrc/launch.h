@@ -42,6 +42,10 @@ hipError_t launch_merge_dev(const MergeArgs *a, int dp, int max_splits, int64_t 
 
 // Merges a.total_items query vectors; max_splits picks the thread layout.
 hipError_t launch_merge(const MergeArgs &a, int dp, int max_splits, hipStream_t stream);
+// Merges `lanes` (decode rows, of up to lane_splits splits) and `few` (prefill rows) of one
+// row group, in one launch where their layouts fit into one.
+hipError_t launch_merge_both(const MergeArgs &lanes, const MergeArgs &few, int dp, int lane_splits, int few_splits,
+                             hipStream_t stream);
 // Splits per query vector up to which the merge gives each (vector, 4
 // features) one thread that folds the splits in increasing order.  The decode
 // kernel's in-launch merge serves only such launches and folds the same way.

@@ -19,8 +19,8 @@
 // decode rows) a block holds FS feature lanes of one vector and SG = THREADS /
 // FS split lanes: all FC feature lanes up to kMergeSliceSplits splits, past
 // that a slice of them, the FC / FS slices of a vector being separate blocks,
-// so a very long row's records are read by many CUs at once.  THREADS (256 to
-// 1024) is chosen so that a lane loads at most one batch of 16 records.
+// so a very long row's records are read by many CUs at once; THREADS (256 or
+// 512) is then chosen so that a lane loads at most one batch of 16 records.
 //
 // Blocks are dealt to the 8 XCDs in contiguous runs of work groups (block b
 // runs group (b % 8) * (grid / 8) + b / 8), the order the prefill kernel
@@ -40,6 +40,20 @@ constexpr int kMergeTile = 128;
 template <int FS, int SG>
 using MergeRed = MergeState[SG > 1 ? SG : 1][SG > 1 ? FS : 1];
 
+// Feature lanes per block past kMergeSliceSplits splits: 64 features, 256
+// contiguous bytes of each record.  Measured on MI355X: slicing takes a
+// 16384-key D = 256 row's merge from 10.3 to 7.2 us at 256 splits and from
+// 6.5 to 5.9 us at 128, and makes merges of 17 to 52 splits 0.2-0.8 us
+// slower than one block per vector.
+constexpr int kMergeSliceLanes = 16;
+constexpr int kMergeSliceSplits = 64;
+
+// Records a lane loads before it folds any: few with one thread for all splits (registers
+// for more waves), all of its splits up to kMergeSliceSplits, else 16.
+constexpr int merge_inflight(int split_lanes, int slices) {
+  return split_lanes == 1 ? 4 : (slices == 1 ? kMergeSliceSplits / split_lanes : 16);
+}
+
 constexpr MergeState kMergeStart{-INFINITY, 0.0f, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
 
 // Folds records first, first + SG, ... below nsplit of one query vector into st over
@@ -50,12 +64,11 @@ constexpr MergeState kMergeStart{-INFINITY, 0.0f, f32x4{0.0f, 0.0f, 0.0f, 0.0f}}
 // f is the thread's feature lane within the block's FS.  Every record of a
 // batch is loaded before any is folded: a lane's splits take
 // ceil(nsplit / (SG * INFLIGHT)) memory round trips.
-template <int FS, int SG>
+template <int FS, int SG, int INFLIGHT>
 __device__ __forceinline__ void fold_and_write(MergeRed<FS, SG> &red, const float *part_o, const float *part_ml,
                                                int64_t o_base, int64_t o_step, int64_t ml_base, int64_t ml_step,
                                                int nsplit, bool active, int sg, int f, uint16_t *dst, MergeState st,
                                                int first) {
-  constexpr int INFLIGHT = SG > 1 ? 16 : 4;
   if (active) {
     for (int s0 = first; s0 < nsplit; s0 += INFLIGHT * SG) {
       u32x2 ml[INFLIGHT];
@@ -94,11 +107,29 @@ __device__ __forceinline__ void fold_and_write(MergeRed<FS, SG> &red, const floa
       u32x2{pack_bf16x2(st.o.x * inv, st.o.y * inv), pack_bf16x2(st.o.z * inv, st.o.w * inv)};
 }
 
-// The kernel's body, shared by the launch with host-planned arguments
-// (merge_kernel) and the graph-capture launch that reads them from device
-// memory (merge_dev_kernel).
+// Every argument of a block, loaded in one round trip (see XATTN_PIN_VIEW).
+struct MergeLocals {
+  RowLookup<MergeRow> rows;
+  int total_items, lane_items, nrows, D, G;
+  uint16_t *out;
+  int64_t o_sb, o_sh, o_st;
+  const float *part_o, *part_ml;
+  __device__ __forceinline__ explicit MergeLocals(const MergeArgs &a)
+      : total_items(a.total_items), lane_items(a.lane_items), nrows(a.nrows), D(a.D), G(a.G), out(a.out),
+        o_sb(a.o_sb), o_sh(a.o_sh), o_st(a.o_st), part_o(a.part_o), part_ml(a.part_ml) {
+    rows.load(a.rows);
+    asm volatile(""
+                 : XATTN_PIN_BEGINS(rows), XATTN_PIN_MERGEROW(rows.first), "+s"(total_items), "+s"(lane_items),
+                   "+s"(nrows), "+s"(D), "+s"(G), "+s"(out), "+s"(o_sb), "+s"(o_sh), "+s"(o_st), "+s"(part_o),
+                   "+s"(part_ml));
+  }
+};
+
+// Block `block` of those that merge vectors first .. end - 1: shared by the launches
+// with host-planned arguments (merge_kernel, merge_both_kernel) and the
+// graph-capture launch that reads them from device memory (merge_dev_kernel).
 template <int DP, int SG, int THREADS, int FS, bool DEV>
-__device__ __forceinline__ void merge_body(const MergeArgs &a) {
+__device__ __forceinline__ void merge_body(const MergeArgs &a, const MergeLocals &l, int block, int first, int end) {
   constexpr int FC = DP / 4;                         // feature lanes of a vector
   static_assert(SG == 1 ? FS == FC : FS * SG == THREADS, "block shape");
   constexpr int NS = FC / FS;                        // feature slices per vector (SG > 1)
@@ -111,30 +142,20 @@ __device__ __forceinline__ void merge_body(const MergeArgs &a) {
   const int tid = threadIdx.x;
   const int fl = SG > 1 ? tid % FS : tid / VPB, sg = SG > 1 ? tid / FS : 0;
   const int vl = VPB == 1 ? 0 : tid % VPB;
-  // Every argument of the block, loaded in one round trip (see XATTN_PIN_VIEW).
-  RowLookup<MergeRow> rows;
-  rows.load(a.rows);
-  int total_items = a.total_items, nrows = a.nrows, D = a.D, G = a.G;
-  uint16_t *out = a.out;
-  int64_t o_sb = a.o_sb, o_sh = a.o_sh, o_st = a.o_st;
-  const float *part_o = a.part_o, *part_ml = a.part_ml;
-  asm volatile(""
-               : XATTN_PIN_BEGINS(rows), XATTN_PIN_MERGEROW(rows.first), "+s"(total_items), "+s"(nrows), "+s"(D),
-                 "+s"(G), "+s"(out), "+s"(o_sb), "+s"(o_sh), "+s"(o_st), "+s"(part_o), "+s"(part_ml));
   // Work groups: VPB vectors (few splits) or one slice of one vector.  The
-  // grid is the groups rounded up to a multiple of 8 (launch_merge_d).
-  const int groups = SG > 1 ? total_items * NS : (total_items + VPB - 1) / VPB;
+  // blocks are the groups rounded up to a multiple of 8 (launch_merge_d).
+  const int groups = SG > 1 ? (end - first) * NS : (end - first + VPB - 1) / VPB;
   // A grid sized for more groups (device-planned launches) leaves surplus blocks.
   if constexpr (DEV) {
-    if ((int)(blockIdx.x / 8) >= (groups + 7) / 8) return;
+    if (block / 8 >= (groups + 7) / 8) return;
   }
-  const int group = (int)(blockIdx.x % 8) * ((groups + 7) / 8) + (int)(blockIdx.x / 8);
-  const int vec = SG > 1 ? group / NS : group * VPB + vl;
-  const int f = SG > 1 ? (group - vec * NS) * FS + fl : fl;  // feature lane of the vector
-  const bool vvalid = vec < total_items;
-  const MergeRow mr = rows.template find<(SG > 1)>(a.rows, nrows, vvalid ? vec : 0);
+  const int group = block % 8 * ((groups + 7) / 8) + block / 8;
+  const int vec = first + (SG > 1 ? group / NS : group * VPB + vl);
+  const int f = SG > 1 ? (group - (vec - first) * NS) * FS + fl : fl;  // feature lane of the vector
+  const bool vvalid = vec < end;
+  const MergeRow mr = l.rows.template find<(SG > 1)>(a.rows, l.nrows, vvalid ? vec : first);
   const int local = vec - mr.item_begin;
-  const int qrows = mr.count * G;
+  const int D = l.D, G = l.G, qrows = mr.count * G;
   const int h = local / qrows, j = local - h * qrows;
   const int d = f * 4;
   // Record s of this vector: o at part_o + o_base + s * o_step, (m, l) at
@@ -155,26 +176,28 @@ __device__ __forceinline__ void merge_body(const MergeArgs &a) {
   }
 
   const int g = j % G, i = j / G;
-  fold_and_write<FS, SG>(red, part_o, part_ml, o_base, o_step, ml_base, ml_step, mr.nsplit, vvalid && d < D, sg, fl,
-                         out + mr.batch * o_sb + (int64_t)(h * G + g) * o_sh + (int64_t)i * o_st + d, kMergeStart, sg);
+  fold_and_write<FS, SG, merge_inflight(SG, NS)>(red, l.part_o, l.part_ml, o_base, o_step, ml_base, ml_step, mr.nsplit, vvalid && d < D, sg, fl,
+                         l.out + mr.batch * l.o_sb + (int64_t)(h * G + g) * l.o_sh + (int64_t)i * l.o_st + d,
+                         kMergeStart, sg);
 }
 
-// Feature lanes per block past kMergeSliceSplits splits: 64 features, 256
-// contiguous bytes of each record.  Measured on MI355X: slicing takes a
-// 16384-key D = 256 row's merge from 10.3 to 7.2 us at 256 splits and from
-// 6.5 to 5.9 us at 128, and makes merges of 17 to 52 splits 0.2-0.8 us
-// slower than one block per vector.
-constexpr int kMergeSliceLanes = 16;
-constexpr int kMergeSliceSplits = 64;
+// Threads of a block with one thread for all splits: 8 vectors per block for
+// D = 256, so that a wave's load reads whole 128-byte lines of the prefill record
+// layout (cfg5's merge 3 us faster than with 4 vectors and half lines; same
+// outputs).
+template <int DP>
+constexpr int kMergeSerialThreads = DP == 256 ? 512 : 256;
 
 template <int DP, int SG, int THREADS, int FS>
 __global__ void __launch_bounds__(THREADS) merge_kernel(const MergeArgs a) {
-  merge_body<DP, SG, THREADS, FS, false>(a);
+  const MergeLocals l(a);
+  merge_body<DP, SG, THREADS, FS, false>(a, l, blockIdx.x, 0, l.total_items);
 }
 
 template <int DP, int SG, int THREADS, int FS>
 __global__ void __launch_bounds__(THREADS) merge_dev_kernel(const MergeArgs *__restrict__ a) {
-  merge_body<DP, SG, THREADS, FS, true>(*a);
+  const MergeLocals l(*a);
+  merge_body<DP, SG, THREADS, FS, true>(*a, l, blockIdx.x, 0, l.total_items);
 }
 
 // The merge's launch: host arguments `a`, or (DEV) the arguments at `dev`;
@@ -193,22 +216,12 @@ static hipError_t launch_merge_d(const MergeArgs &a, const MergeArgs *dev, int m
   constexpr int FC = DP / 4;
   // Grids are rounded up to a multiple of the 8 XCDs; surplus groups exit.
   if (max_splits <= kMergeSerialSplits) {
-    // 8 vectors per block for D = 256 (512 threads), so that a wave's load
-    // reads whole 128-byte lines of the prefill record layout (cfg5's merge
-    // 3 us faster than with 4 vectors and half lines; same outputs).
-    constexpr int THREADS = DP == 256 ? 512 : 256;
+    constexpr int THREADS = kMergeSerialThreads<DP>;
     constexpr int VPB = THREADS / FC;
     launch_merge_kernel<DP, 1, THREADS, FC, DEV>(dim3(((vectors + VPB - 1) / VPB + 7) / 8 * 8), a, dev, stream);
   } else if (max_splits <= kMergeSliceSplits) {
-    // One block per vector, with enough split lanes that each lane loads at
-    // most one batch of 16 records when the block can grow to 1024 threads.
-    const dim3 grid((vectors + 7) / 8 * 8);
-    if (max_splits <= 16 * (256 / FC))
-      launch_merge_kernel<DP, 256 / FC, 256, FC, DEV>(grid, a, dev, stream);
-    else if (max_splits <= 16 * (512 / FC))
-      launch_merge_kernel<DP, 512 / FC, 512, FC, DEV>(grid, a, dev, stream);
-    else
-      launch_merge_kernel<DP, 1024 / FC, 1024, FC, DEV>(grid, a, dev, stream);
+    // One block per vector: a lane loads its splits in one batch.
+    launch_merge_kernel<DP, 256 / FC, 256, FC, DEV>(dim3((vectors + 7) / 8 * 8), a, dev, stream);
   } else {
     // One block per (vector, slice of FS feature lanes).
     constexpr int FS = FC < kMergeSliceLanes ? FC : kMergeSliceLanes;
@@ -266,7 +279,7 @@ __global__ void __launch_bounds__(256) merge_capture_kernel(const CaptureArgs c)
       if (sg + u * SG < nsplit) fold(st, __uint_as_float(ml[u].x), __uint_as_float(ml[u].y), o[u]);
   }
   const int g = j % c.G, i = j / c.G;
-  fold_and_write<FC, SG>(red, c.part_o, c.part_ml, o_base, o_step, ml_base, ml_step, nsplit, d < c.D, sg, f,
+  fold_and_write<FC, SG, 16>(red, c.part_o, c.part_ml, o_base, o_step, ml_base, ml_step, nsplit, d < c.D, sg, f,
                          c.out + r * c.o_sb + (int64_t)(h * c.G + g) * c.o_sh + (int64_t)i * c.o_st + d, st,
                          ahead ? sg + AHEAD * SG : sg);
 }
@@ -286,6 +299,50 @@ hipError_t launch_merge(const MergeArgs &a, int dp, int max_splits, hipStream_t 
     case 64: return launch_merge_d<64, false>(a, nullptr, max_splits, a.total_items, stream);
     case 128: return launch_merge_d<128, false>(a, nullptr, max_splits, a.total_items, stream);
     default: return launch_merge_d<256, false>(a, nullptr, max_splits, a.total_items, stream);
+  }
+}
+
+// The rows of many splits (decode) and those of few (prefill) of a mixed batch in
+// one launch: the first round8(lane_items) blocks take one vector each, the others
+// several.  (A mixed step of 7 decode rows and a 384-token prefill row, D = 128: one launch
+// of 5.7 us in place of two of 4.7 and 4.5, the step 45.6 -> 42.9 us.)
+template <int DP>
+__global__ void __launch_bounds__(kMergeSerialThreads<DP>) merge_both_kernel(const MergeArgs a) {
+  constexpr int THREADS = kMergeSerialThreads<DP>, FC = DP / 4;
+  const MergeLocals l(a);
+  const int lane_blocks = (l.lane_items + 7) / 8 * 8, block = blockIdx.x;
+  if (block < lane_blocks) merge_body<DP, THREADS / FC, THREADS, FC, false>(a, l, block, 0, l.lane_items);
+  else merge_body<DP, 1, THREADS, FC, false>(a, l, block - lane_blocks, l.lane_items, l.total_items);
+}
+
+template <int DP>
+static hipError_t launch_merge_both_d(const MergeArgs &a, hipStream_t stream) {
+  constexpr int THREADS = kMergeSerialThreads<DP>, VPB = THREADS / (DP / 4);
+  const int few = (a.total_items - a.lane_items + VPB - 1) / VPB;
+  hipLaunchKernelGGL(merge_both_kernel<DP>, dim3((a.lane_items + 7) / 8 * 8 + (few + 7) / 8 * 8), dim3(THREADS), 0,
+                     stream, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_merge_both(const MergeArgs &lanes, const MergeArgs &few, int dp, int lane_splits, int few_splits,
+                             hipStream_t stream) {
+  if (few_splits > kMergeSerialSplits || lane_splits > kMergeSliceSplits) {
+    const hipError_t rc = launch_merge(lanes, dp, lane_splits, stream);
+    return rc != hipSuccess ? rc : launch_merge(few, dp, few_splits, stream);
+  }
+  MergeArgs both = lanes;
+  both.lane_items = lanes.total_items;
+  both.total_items += few.total_items;
+  for (int r = 0; r < few.nrows; ++r) {
+    MergeRow &row = both.rows[both.nrows++];  // rows of one group: at most kMaxRows
+    row = few.rows[r];
+    row.item_begin += lanes.total_items;
+  }
+  if (lane_splits <= kMergeSerialSplits) return launch_merge(both, dp, kMergeSerialSplits, stream);
+  switch (dp) {
+    case 64: return launch_merge_both_d<64>(both, stream);
+    case 128: return launch_merge_both_d<128>(both, stream);
+    default: return launch_merge_both_d<256>(both, stream);
   }
 }
 
