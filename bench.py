@@ -81,9 +81,8 @@ def dominant_kernel(w):
     Mirrors the library's kernel choice: head dims pad to 64 / 128 / 256;
     prefill runs two waves per query group (8 waves) at 64 and 128 and the
     kernel of its own at 256 (a plain function, so its demangled name carries
-    no return type); decode is instantiated for the power-of-two query vectors
-    per KV head (count * G) and the rounds per item, four when one-round items
-    would number at least 1536 (the planner in capi.cpp), else one.
+    no return type); decode is instantiated for one or two groups of 16 columns,
+    of which a query vector takes three up to 8 of them per KV head (count * G), else one.
     """
     dp = 64 if w.dim <= 64 else (128 if w.dim <= 128 else 256)
     if w.kind == "prefill":
@@ -92,14 +91,8 @@ def dominant_kernel(w):
         return f"void xattn::prefill_kernel<{dp}, 2>(xattn::AttnArgs)"
     group = w.heads // w.kv_heads
     qv = max(1, max(c for c in w.counts) * group)
-    qr = 1
-    while qr < qv:
-        qr *= 2
-    keys_per_round = (16384 if qr <= 4 else 8192) // dp
-    one_round_items = sum(w.kv_heads * -(-length // keys_per_round)
-                          for count, length in zip(w.counts, w.lengths) if count > 0)
-    rounds = 4 if one_round_items >= 1536 else 1
-    return f"void xattn::decode_kernel<{dp}, {qr}, {rounds}>(xattn::AttnArgs)"
+    groups = 1 if 3 * qv <= 16 or 8 < qv <= 16 else 2
+    return f"void xattn::decode_kernel<{dp}, {groups}>(xattn::AttnArgs)"
 
 
 def record_traffic(fetch_csv, write_csv):

@@ -28,6 +28,8 @@ def check(gpu_ops, heads, kv_heads, dim, counts, lengths, capacity):
     expected = oracle.attention(f64(q), f64(k), f64(v), counts, lengths, dim ** -0.5)
     for r, count in enumerate(counts):
         assert torch.count_nonzero(out[r, :, count:]).item() == 0
+        if count == 0:
+            continue
         errors = row_errors(out[r:r + 1, :, :count].float().flatten(1),
                             torch.from_numpy(expected[r:r + 1, :, :count]).float().flatten(1))
         assert errors["max_abs"] <= MAX_ABS and errors["mean_abs"] <= MEAN_ABS, (r, errors)
@@ -53,3 +55,15 @@ def test_decode_and_prefill_rows_merge_together(gpu_ops, dim):
     counts, lengths = [1, 40, 2, 33, 1, 65], [3000, 2900, 2400, 1500, 700, 513]
     log(f"merge of both kinds D={dim} counts={counts} lengths={lengths}")
     check(gpu_ops, 12, 3, dim, counts, lengths, 3001)
+
+
+@pytest.mark.parametrize("dim", (64, 72, 128, 256))
+@pytest.mark.parametrize("counts,lengths", [
+    ([0, 96, 1, 1, 5, 130], [9, 900, 1, 700, 200, 1301]),  # one launch; an odd number of decode items, a row without queries
+    ([1, 1, 70], [40, 33, 70]),                            # one item a head, no splits
+    ([1] * 40 + [40] * 3, [1100] * 40 + [50, 60, 70]),     # two launches: the decode rows take longer
+])
+@torch.inference_mode()
+def test_decode_and_prefill_rows_launch_together(gpu_ops, dim, counts, lengths):
+    log(f"launch of both kinds D={dim} counts={counts} lengths={lengths}")
+    check(gpu_ops, 6, 3, dim, counts, lengths, 1303)

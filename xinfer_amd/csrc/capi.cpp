@@ -78,6 +78,7 @@ struct Group {
   int dec_merge_items = 0, pre_merge_items = 0, pre_max_splits = 1;
   // The decode launch may merge its split rows itself (decode_merge_fusable).
   bool dec_fusable = false;
+  bool both = false;  // decode and prefill rows in one launch (one_launch_pays)
 };
 
 struct Plan {
@@ -475,6 +476,37 @@ int64_t decode_vector_limit(const Geometry &g, const std::vector<int32_t> &count
   return wide && !narrow && keys <= kShortRowKeys ? kExactVectors : kStreamMaxVectors;
 }
 
+// Whether the decode rows `dec` and the prefill rows whose items take `work`
+// microseconds go in one launch, where decode items stream their keys on the CUs
+// that the prefill items leave free or have left.  An item pair per CU streams less
+// well than two independent blocks, so it pays where prefill items leave CUs free
+// (at most 3/4 of the CUs have one) while the decode rows' bytes (keys, and zeros of
+// padded queries) take no longer than the prefill items, up to 2.6 times as
+// long for head dims 64 and 256; where they fill the chip, only for a few decode rows
+// beside long prefill.  Measured, two launches -> one (us; ratio of the two times):
+// few prefill items: D = 128: 7 decode rows and 384 tokens 32.8 -> 24.6 (0.8), 6 rows of 6
+// and 256 tokens 32.2 -> 23.3 (0.8); D = 256: 7 rows and 300 tokens 45.7 -> 32.5 (0.6),
+// 7 long rows 77.7 -> 67.5 (2.5); D = 64: 24.9 -> 16.2 (0.4), 20 rows 38.7 -> 33.1 (2.0).
+// Many: D = 128: 4 rows and 4 x 512 tokens 174 -> 162 (0.1), 1 row and 2000 tokens 198 -> 191
+// (0.04), but 6 rows and 4 x 512 tokens 128 -> 131 (0.2), 5 rows and 512 tokens 36.9 -> 39.2
+// (0.9), 7 long rows 45.2 -> 53.5 (1.8), 31 long rows and 4 x 512 tokens 187 -> 211 (0.7);
+// D = 64 109 -> 126 (0.8).
+bool one_launch_pays(const Geometry &g, const AttnArgs &dec, int G, int dp, const std::vector<double> &work) {
+  double bytes = 0, total = 0, longest = 0;
+  for (int r = 0; r < dec.nrows; ++r) {
+    const RowSched &rs = dec.rows[r];
+    if (rs.count > 0) bytes += 4.0 * (double)rs.length * (double)(g.Hkv * g.D);
+    bytes += 2.0 * (double)(g.T - rs.count) * (double)(g.Hkv * G * g.D);
+  }
+  for (const double us : work) {
+    total += us;
+    longest = std::max(longest, us);
+  }
+  const double prefill_us = std::max(longest, total / (8.0 * kCusPerXcd));
+  const bool free_cus = work.size() <= 8 * kCusPerXcd * 3 / 4;
+  return bytes / kDecodeBytesPerUs <= (free_cus ? (dp == 128 ? 1.0 : 2.6) : 0.1) * prefill_us;
+}
+
 // counts/lengths: per-row real queries and populated KV lengths (validated).
 Plan make_plan(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths) {
   Plan plan;
@@ -553,7 +585,11 @@ Plan make_plan(const Geometry &g, const std::vector<int32_t> &counts, const std:
     plan.records = std::max(plan.records, records);
     grp.dec_fusable = decode_merge_fusable(grp, g.Hkv) && !(prefill_split && !choice.sized);
     if (grp.dec_fusable) plan.counters = std::max<int64_t>(plan.counters, grp.dec_items);
-    if (grp.pre_items > 0) xcd_runs(prefill_item_work(grp.pre.rows, grp.pre.nrows, g.Hkv, G, dp), grp.pre.xcd_begin);
+    if (grp.pre_items > 0) {
+      const std::vector<double> work = prefill_item_work(grp.pre.rows, grp.pre.nrows, g.Hkv, G, dp);
+      xcd_runs(work, grp.pre.xcd_begin);
+      if (grp.dec_items > 0) grp.both = one_launch_pays(g, grp.dec, G, dp, work);
+    }
     plan.groups.push_back(grp);
   }
   return plan;
@@ -628,15 +664,20 @@ int run_plan(const Plan &plan, const Geometry &g, const xinfer_view4 &q, const x
     grp.pre.total_items = grp.pre_items;
     grp.dec.arrive_ctr = nullptr;
     grp.dec.tag = 0;
-    if (grp.dec_fusable && !merge_launch_forced() && decode_merge_in_launch_pays(grp.dec_items) &&
+    if (!grp.both && grp.dec_fusable && !merge_launch_forced() && decode_merge_in_launch_pays(grp.dec_items) &&
         xcd_dispatch_round_robin(stream)) {
       grp.dec.arrive_ctr = reinterpret_cast<uint64_t *>(static_cast<char *>(workspace) + plan.counters_offset());
       grp.dec.tag = next_launch_tag();
       grp.dec_merge_items = 0;  // the decode rows are merged in the launch
     }
-    if (grp.dec_items > 0 && launch_decode(grp.dec, dp, grp.dec_columns, grp.dec_items, stream) != hipSuccess)
-      return XINFER_ERR_LAUNCH;
-    if (grp.pre_items > 0 && launch_prefill(grp.pre, dp, stream) != hipSuccess) return XINFER_ERR_LAUNCH;
+    hipError_t rc = hipSuccess;
+    if (grp.both) {
+      rc = launch_attention_both(grp.dec, grp.pre, dp, grp.dec_columns, stream);
+    } else {
+      if (grp.dec_items > 0) rc = launch_decode(grp.dec, dp, grp.dec_columns, grp.dec_items, stream);
+      if (rc == hipSuccess && grp.pre_items > 0) rc = launch_prefill(grp.pre, dp, stream);
+    }
+    if (rc != hipSuccess) return XINFER_ERR_LAUNCH;
     grp.dec_merge.total_items = grp.dec_merge_items;
     grp.pre_merge.total_items = grp.pre_merge_items;
     for (MergeArgs *m : {&grp.dec_merge, &grp.pre_merge}) {
@@ -649,7 +690,6 @@ int run_plan(const Plan &plan, const Geometry &g, const xinfer_view4 &q, const x
       m->D = (int32_t)g.D;
       m->G = G;
     }
-    hipError_t rc = hipSuccess;
     if (grp.dec_merge_items > 0 && grp.pre_merge_items > 0)
       rc = launch_merge_both(grp.dec_merge, grp.pre_merge, dp, grp.dec_max_splits, grp.pre_max_splits, stream);
     else if (grp.dec_merge_items > 0)

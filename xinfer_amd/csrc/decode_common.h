@@ -321,6 +321,13 @@ struct WaveAttention {
   }
 };
 
+// Passes of combine_waves, and its barriers: 2 * passes - 1.
+template <int DP, int NC, int BYTES>
+constexpr int combine_passes() {
+  using S = DecodeShape<DP, NC>;
+  return S::DT * NC * 1024 > BYTES ? S::DT * NC * 1024 / BYTES : 1;
+}
+
 // Combines the states of a block's WAVES waves and hands every query vector's
 // quads of features to write(j, d, o, m, l) (features d .. d+3 of vector j, the
 // unnormalised sum, the running max and the normaliser).  Wave w's state goes
@@ -330,11 +337,11 @@ struct WaveAttention {
 // banks.  red_ml holds [wave][column] (m, l).
 template <int DP, int NC, int WAVES, int BYTES, typename Write>
 __device__ __forceinline__ void combine_waves(const WaveAttention<DP, NC> &w, char *states, float2 *red_ml, int qrows,
-                                              int D, int wave, Write &&write) {
+                                              int D, int tid, int wave, Write &&write) {
   using S = DecodeShape<DP, NC>;
-  constexpr int PASSES = S::DT * NC * 1024 > BYTES ? S::DT * NC * 1024 / BYTES : 1;
+  constexpr int PASSES = combine_passes<DP, NC, BYTES>();
   constexpr int DTP = S::DT / PASSES, FQ = DTP * 4;  // d tiles and feature quads of a pass
-  const int tid = threadIdx.x, col = w.col, grp = w.grp;
+  const int col = w.col, grp = w.grp;
 #pragma unroll
   for (int pass = 0; pass < PASSES; ++pass) {
     if (pass > 0) __syncthreads();

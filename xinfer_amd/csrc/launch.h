@@ -30,6 +30,10 @@ hipError_t launch_decode(const AttnArgs &a, int dp, int columns, int items, hipS
 hipError_t launch_prefill(const AttnArgs &a, int dp, hipStream_t stream);
 // The head-dim-256 prefill kernel over `blocks` blocks (prefill_d256.hip).
 hipError_t launch_prefill_d256(const AttnArgs &a, unsigned blocks, hipStream_t stream);
+// The decode rows (without a merge in the launch) and the prefill rows of one row group in
+// one launch.
+hipError_t launch_attention_both(const AttnArgs &dec, const AttnArgs &pre, int dp, int columns, hipStream_t stream);
+hipError_t launch_attention_both_d256(const AttnArgs &a, int columns, dim3 grid, hipStream_t stream);
 // Graph-capture prefill: the plan kernel writes *p.attn and *p.merge from the
 // device offsets, then the prefill kernel runs over `blocks` blocks with its
 // arguments read from *p.attn (blocks past their XCD run exit).

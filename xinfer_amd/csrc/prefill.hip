@@ -49,6 +49,9 @@
 // Several splits of a tile write fp32 partial records, combined by merge.hip;
 // a tile's records per split are laid out [D/4][128 vectors][4 features].
 // The tile-0 / split-0 item zeroes the row's padded queries (t >= count).
+#include <algorithm>
+
+#include "decode_item.h"
 #include "launch.h"
 #include "prefill_common.h"
 
@@ -81,13 +84,23 @@ struct PrefillShape {
 // The kernel's body, shared by the launch with host-planned arguments
 // (prefill_kernel) and the graph-capture launch that reads them from device
 // memory (prefill_dev_kernel).
-template <int DP, int KH, bool DEV>
+//
+// NC > 0: blocks y = 1 of the launch take two decode items each instead, of NC
+// column groups (attention_both_kernel).
+template <int DP, int KH, bool DEV, int NC = 0>
 __device__ __forceinline__ void prefill_body(const AttnArgs &a) {
   using S = PrefillShape<DP, KH>;
   constexpr int THREADS = S::THREADS, NDS = S::NDS, NDT = S::NDT, CHUNKS = S::CHUNKS;
   constexpr int TILE = S::TILE, LOADS = S::LOADS, NST = S::NST, KPW = S::KPW, NKT = S::NKT;
   static_assert(LOADS >= 1 && S::BN * CHUNKS == LOADS * THREADS, "tile = whole load instructions");
-  __shared__ __attribute__((aligned(16))) uint16_t smem[S::SMEM / 2];
+  constexpr int DECODE = NC > 0 ? 2 * ItemShared<DP, NC ? NC : 1>::BYTES : 0;
+  __shared__ __attribute__((aligned(16))) uint16_t smem[(S::SMEM > DECODE ? S::SMEM : DECODE) / 2];
+  if constexpr (NC > 0) {
+    if (blockIdx.y == 1) {
+      decode_pair<DP, NC>(a, blockIdx.x, reinterpret_cast<char *>(smem));
+      return;
+    }
+  }
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int col = lane & 31, half = lane >> 5;
@@ -462,6 +475,17 @@ __global__ void __launch_bounds__(256 * KH) prefill_dev_kernel(const AttnArgs *_
   prefill_body<DP, KH, true>(*a);
 }
 
+// The prefill and the decode rows of a mixed batch in one launch: blocks y = 0 take
+// the prefill items, blocks y = 1, which are dispatched after them, two decode
+// items each.  Prefill items are bound by matrix and vector work, decode items by
+// HBM, and neither kind alone fills the chip in a step of a few rows: a mixed step
+// of 7 decode rows and a 384-token row, whose two launches took 15 us each, went
+// from 42.9 to 35.6 us (when it is used: capi.cpp: one_launch_pays).
+template <int DP, int NC>
+__global__ void __launch_bounds__(512) attention_both_kernel(const AttnArgs a) {
+  prefill_body<DP, 2, false, NC>(a);
+}
+
 // ceil(a / b) for 0 <= a, 0 < b < 2^31.
 __device__ __forceinline__ int plan_ceil_div(int a, int b) {
   return (int)(((unsigned)a + (unsigned)b - 1u) / (unsigned)b);
@@ -731,18 +755,41 @@ hipError_t launch_prefill_capture(const PrefillPlanArgs &p, int dp, unsigned blo
 
 // Blocks per launch: 8 times the longest XCD run (blocks past their run exit
 // at once).
-hipError_t launch_prefill(const AttnArgs &a, int dp, hipStream_t stream) {
+// Blocks of a prefill launch: the XCDs take turns.
+static unsigned prefill_blocks(const AttnArgs &a) {
   int longest = 0;
-  for (int x = 0; x < 8; ++x) {
-    const int run = a.xcd_begin[x + 1] - a.xcd_begin[x];
-    longest = run > longest ? run : longest;
-  }
-  const dim3 grid(8 * longest);
+  for (int x = 0; x < 8; ++x) longest = std::max(longest, a.xcd_begin[x + 1] - a.xcd_begin[x]);
+  return 8u * longest;
+}
+
+hipError_t launch_prefill(const AttnArgs &a, int dp, hipStream_t stream) {
+  const dim3 grid(prefill_blocks(a));
   switch (dp) {
     case 64: hipLaunchKernelGGL((prefill_kernel<64, 2>), grid, dim3(512), 0, stream, a); break;
     case 128: hipLaunchKernelGGL((prefill_kernel<128, 2>), grid, dim3(512), 0, stream, a); break;
     default: return launch_prefill_d256(a, grid.x, stream);
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_attention_both(const AttnArgs &dec, const AttnArgs &pre, int dp, int columns, hipStream_t stream) {
+  AttnArgs both = pre;
+  both.total_items = dec.total_items;  // decode items; the prefill items follow
+  both.nrows = 0;
+  for (int r = 0; r < dec.nrows; ++r) both.rows[both.nrows++] = dec.rows[r];
+  for (int r = 0; r < pre.nrows; ++r) {  // rows of one group: at most kMaxRows
+    RowSched &row = both.rows[both.nrows++];
+    row = pre.rows[r];
+    row.item_begin += dec.total_items;
+  }
+  for (int &begin : both.xcd_begin) begin += dec.total_items;
+  const unsigned pairs = (dec.total_items + 1) / 2;
+  const dim3 grid(std::max(prefill_blocks(pre), (pairs + 7) / 8 * 8), 2);
+  if (dp == 256) return launch_attention_both_d256(both, columns, grid, stream);
+  if (dp == 64 && columns == 1) hipLaunchKernelGGL((attention_both_kernel<64, 1>), grid, dim3(512), 0, stream, both);
+  else if (dp == 64) hipLaunchKernelGGL((attention_both_kernel<64, 2>), grid, dim3(512), 0, stream, both);
+  else if (columns == 1) hipLaunchKernelGGL((attention_both_kernel<128, 1>), grid, dim3(512), 0, stream, both);
+  else hipLaunchKernelGGL((attention_both_kernel<128, 2>), grid, dim3(512), 0, stream, both);
   return hipGetLastError();
 }
 

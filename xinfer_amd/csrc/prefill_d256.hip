@@ -38,6 +38,7 @@
 // K/V tiles travel HBM -> LDS through buffer_load ... lds over a ring of four
 // 32 KB stages (K and V of a tile): tile t is read in steps t (K) and t+1
 // (V), so step s issues the loads of tile s+2 into the stage of tile s-2.
+#include "decode_item.h"
 #include "launch.h"
 #include "prefill_common.h"
 
@@ -62,9 +63,17 @@ static_assert(kSmemBytes <= 160 * 1024, "LDS");
 
 // The kernel's body, shared by the launch with host-planned arguments and
 // the graph-capture launch that reads them from device memory.
-template <bool DEV>
+// NC > 0: blocks y = 1 of the launch take two decode items each instead.
+template <bool DEV, int NC = 0>
 __device__ __forceinline__ void prefill_d256_body(const AttnArgs &a) {
-  __shared__ __attribute__((aligned(16))) uint16_t smem[kSmemBytes / 2];
+  constexpr int DECODE = NC > 0 ? 2 * ItemShared<kDP, NC ? NC : 1>::BYTES : 0;
+  __shared__ __attribute__((aligned(16))) uint16_t smem[(kSmemBytes > DECODE ? kSmemBytes : DECODE) / 2];
+  if constexpr (NC > 0) {
+    if (blockIdx.y == 1) {
+      decode_pair<kDP, NC>(a, blockIdx.x, reinterpret_cast<char *>(smem));
+      return;
+    }
+  }
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int col = lane & 31, half = lane >> 5;
   const int qgroup = wave & 3;
@@ -381,8 +390,20 @@ __global__ void __launch_bounds__(kThreads) prefill_d256_dev_kernel(const AttnAr
   prefill_d256_body<true>(*a);
 }
 
+// Prefill and decode rows in one launch, as prefill.hip's attention_both_kernel.
+template <int NC>
+__global__ void __launch_bounds__(kThreads) attention_both_d256_kernel(const AttnArgs a) {
+  prefill_d256_body<false, NC>(a);
+}
+
 hipError_t launch_prefill_d256(const AttnArgs &a, unsigned blocks, hipStream_t stream) {
   hipLaunchKernelGGL(prefill_d256_kernel, dim3(blocks), dim3(kThreads), 0, stream, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_attention_both_d256(const AttnArgs &a, int columns, dim3 grid, hipStream_t stream) {
+  if (columns == 1) hipLaunchKernelGGL(attention_both_d256_kernel<1>, grid, dim3(kThreads), 0, stream, a);
+  else hipLaunchKernelGGL(attention_both_d256_kernel<2>, grid, dim3(kThreads), 0, stream, a);
   return hipGetLastError();
 }
 
