@@ -530,11 +530,15 @@ Plan make_plan(const Geometry &g, const std::vector<int32_t> &counts, const std:
     const DecodeChoice choice = choose_decode(g, counts, lengths, row0, grp.nrows, G, dp, decode_vectors,
                                               g.Hkv % 8 == 0 && !prefill_split);
     int64_t records = 0;  // of this group: the groups' launches run one after another
-    // Longer rows first: the launch's last items are then short ones.
+    // Longer decode rows first: the launch's last items are then short ones.  Prefill
+    // rows keep the batch's order, which choose_split_keys simulates (sorted as
+    // well, a ragged D = 256 batch took 488 us in place of 457).
     std::vector<int> order(grp.nrows);
     std::iota(order.begin(), order.end(), 0);
-    std::stable_sort(order.begin(), order.end(),
-                     [&](int x, int y) { return lengths[row0 + x] > lengths[row0 + y]; });
+    auto decode_length = [&](int r) {
+      return (int64_t)counts[row0 + r] * G <= decode_vectors ? lengths[row0 + r] : 0;
+    };
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return decode_length(x) > decode_length(y); });
     for (const int r : order) {
       const int64_t b = row0 + r;
       const int cnt = counts[b], len = lengths[b];
