@@ -29,7 +29,7 @@ namespace xattn {
 namespace {
 
 constexpr int kCaptureDecodeMaxVectors = 8;  // graph capture: G * T at or below this takes the decode kernel
-constexpr int64_t kDecodeManyItems = 1536;  // one-pass decode items from which items are sized to the chip
+constexpr int64_t kDecodeManyItems = 640;  // one-pass decode items from which items are sized to the chip
 constexpr int kPrefillTileQ = 128;         // query vectors per prefill work item
 constexpr int64_t kPrefillMinSplitKeys = 512;
 
@@ -142,7 +142,10 @@ bool decode_merge_in_launch_pays(int64_t items) {
 // Keys per decode item of rows [row0, row0 + nrows), in whole passes of a
 // block's four waves (decode_tokens_per_item).
 //
-// Launches with at least kDecodeManyItems one-pass items, and those with rows of
+// Launches with at least kDecodeManyItems one-pass items (sized against one-pass
+// items, attention alone: 1400 of them 19.8 / 24.4 us, 1304 19.4 / 23.0, 1520 21.7 / 25.1,
+// about 1000 15.5 / 17.0, D = 256, 700, 14.7 / 18.2; 32 rows of up to 700 keys, about 800,
+// 13.2 / 12.7), and those with rows of
 // more than kExactVectors query vectors (whose records are large) or beside
 // prefill rows, size their items to the chip (sized; kernel_args.h: kDecodeCus).
 // Smaller launches compare, by decode_launch_us, items of one pass against items
