@@ -146,9 +146,11 @@ int xinfer_batched_flash_attention_graph(const xinfer_view4 *q, const xinfer_vie
  * xinfer_batched_flash_attention, bit for bit; the split records go to a
  * static device array of the library (one per GPU, held until the process
  * ends) instead of a caller's workspace, and the call allocates nothing.
- * A call whose records exceed XINFER_NOALLOC_SCRATCH_BYTES (the size
- * xinfer_batched_flash_attention_workspace_size reports) returns
- * XINFER_ERR_SCRATCH and launches nothing.  The current device must be the
+ * A call whose records (the size xinfer_batched_flash_attention_workspace_size
+ * reports) exceed XINFER_NOALLOC_SCRATCH_BYTES splits its rows of up to 32 query
+ * vectors per KV head less, which is slower and rounds differently; if the
+ * other rows' records alone exceed it, the call returns XINFER_ERR_SCRATCH and
+ * launches nothing.  The current device must be the
  * stream's.  Calls that overlap in time on one GPU share its array and race:
  * order them on one stream. */
 #define XINFER_NOALLOC_SCRATCH_BYTES (32u << 20)

@@ -155,12 +155,13 @@ bool decode_merge_in_launch_pays(int64_t items) {
 // seeds 1 and 3, one pass + merge launch against four passes + in-launch merge):
 // 10.2 / 11.9 us and 13.6 / 12.8 us; the model picks the faster of each.
 // vectors: rows of up to that many query vectors per KV head are decode rows.
+// stretch: items that many times as long (make_plan: fewer records).
 struct DecodeChoice {
   bool sized;
   int64_t keys;
 };
 DecodeChoice choose_decode(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths,
-                           int64_t row0, int nrows, int G, int dp, int64_t vectors, bool fusable) {
+                           int64_t row0, int nrows, int G, int dp, int64_t vectors, bool fusable, int64_t stretch) {
   int64_t items[2] = {0, 0}, max_splits[2] = {1, 1}, keys = 0, widest = 0, longest = 1, pairs = 0;
   bool prefill = false;
   const int64_t pass = decode_tokens_per_item(dp);
@@ -206,9 +207,9 @@ DecodeChoice choose_decode(const Geometry &g, const std::vector<int32_t> &counts
     const int64_t m1 = least(kDecodeCus), m2 = least(2 * kDecodeCus);
     int64_t m = 2 * m2 < m1 ? m2 : m1;
     if (!even(m1, kDecodeCus) && !even(m2, 2 * kDecodeCus)) m = least(4 * kDecodeCus);
-    return {true, m * pass};
+    return {true, m * pass * stretch};
   }
-  if (!fusable || max_splits[1] > kMergeSerialSplits) return {false, pass};
+  if (!fusable || max_splits[1] > kMergeSerialSplits) return {false, pass * stretch};
   const double kv_bytes = 4.0 * (double)(keys * g.D);
   double us[2];
   for (int o = 0; o < 2; ++o) {
@@ -216,7 +217,7 @@ DecodeChoice choose_decode(const Geometry &g, const std::vector<int32_t> &counts
     const bool in_launch = max_splits[o] <= kMergeSerialSplits && decode_merge_in_launch_pays(items[o]);
     us[o] = decode_launch_us(items[o], rounds[o], kv_bytes, split, in_launch);
   }
-  return {false, (us[1] < us[0] ? kDecodeItemRounds : 1) * pass};
+  return {false, (us[1] < us[0] ? kDecodeItemRounds : 1) * pass * stretch};
 }
 
 // 64-key tiles of prefill item (split, query tile) of row rs: the key range
@@ -510,14 +511,16 @@ bool one_launch_pays(const Geometry &g, const AttnArgs &dec, int G, int dp, cons
   return bytes / kDecodeBytesPerUs <= (free_cus ? (dp == 128 ? 1.0 : 2.6) : 0.1) * prefill_us;
 }
 
-// counts/lengths: per-row real queries and populated KV lengths (validated).
-Plan make_plan(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths) {
+// The schedule of a call whose rows of up to decode_vectors query vectors per KV
+// head take the decode kernel, its items `stretch` times as long as
+// choose_decode has them.
+Plan plan_rows(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths,
+               int64_t decode_vectors, int64_t stretch) {
   Plan plan;
   plan.D = g.D;
   const int G = (int)(g.Hq / g.Hkv);
   const int dp = padded_dim(g.D);
 
-  const int64_t decode_vectors = decode_vector_limit(g, counts, lengths, G);
   // Keys per prefill split, chosen from the whole call's prefill work.
   const int64_t split_keys = choose_split_keys(g, counts, lengths, G, dp, decode_vectors);
 
@@ -531,7 +534,7 @@ Plan make_plan(const Geometry &g, const std::vector<int32_t> &counts, const std:
       if (qv > decode_vectors && prefill_splits(lengths[row0 + r], split_keys) > 1) prefill_split = true;
     }
     const DecodeChoice choice = choose_decode(g, counts, lengths, row0, grp.nrows, G, dp, decode_vectors,
-                                              g.Hkv % 8 == 0 && !prefill_split);
+                                              g.Hkv % 8 == 0 && !prefill_split, stretch);
     int64_t records = 0;  // of this group: the groups' launches run one after another
     // Longer decode rows first: the launch's last items are then short ones.  Prefill
     // rows keep the batch's order, which choose_split_keys simulates (sorted as
@@ -602,28 +605,52 @@ Plan make_plan(const Geometry &g, const std::vector<int32_t> &counts, const std:
   return plan;
 }
 
+// counts/lengths: per-row real queries and populated KV lengths (validated).
+//
+// max_bytes: what the entry point's own scratch holds (the allocation-free one),
+// where the caller brings no workspace.  A plan that needs more gives way: longer
+// decode items, then rows of more than kExactVectors vectors on the prefill
+// kernel as well, whose records are those of their query tiles.  The last
+// plan tried splits no decode row, so what is refused is refused for prefill
+// records alone.
+Plan make_plan(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths,
+               size_t max_bytes) {
+  const int64_t limit = decode_vector_limit(g, counts, lengths, (int)(g.Hq / g.Hkv));
+  Plan plan = plan_rows(g, counts, lengths, limit, 1);
+  if (plan.bytes() > max_bytes) plan = plan_rows(g, counts, lengths, limit, 2);
+  const int64_t pass = decode_tokens_per_item(padded_dim(g.D));
+  for (int64_t stretch = 1; plan.bytes() > max_bytes; stretch *= 2) {
+    plan = plan_rows(g, counts, lengths, kExactVectors, stretch);
+    if (stretch * pass >= g.C) break;  // every item at least a row's keys
+  }
+  return plan;
+}
+
 // The plan of this thread's last call.  A model step calls the operator once
 // per layer with the same counts and lengths, and every call plans twice (its
 // workspace size, then the launch), while planning a ragged prefill batch
 // simulates its dispatch at several split sizes (about 0.36 ms for the
-// batch-8 D = 256 prefill of 2235 tokens); a call whose geometry, counts and
-// lengths equal the last one's reuses that plan.  A plan depends on nothing
-// else: not on the device, the stream or the tensors' addresses.
-Plan cached_plan(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths) {
+// batch-8 D = 256 prefill of 2235 tokens); a call whose geometry, counts,
+// lengths and record limit equal the last one's reuses that plan.  A plan depends
+// on nothing else: not on the device, the stream or the tensors' addresses.
+Plan cached_plan(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths,
+                 size_t max_bytes = SIZE_MAX) {
   struct Entry {
     bool valid = false;
+    size_t max_bytes = 0;
     Geometry g{};
     std::vector<int32_t> counts, lengths;
     Plan plan;
   };
   thread_local Entry last;
   const bool same = last.valid && last.g.B == g.B && last.g.Hq == g.Hq && last.g.Hkv == g.Hkv &&
-                    last.g.T == g.T && last.g.D == g.D && last.g.C == g.C && last.counts == counts &&
-                    last.lengths == lengths;
+                    last.g.T == g.T && last.g.D == g.D && last.g.C == g.C && last.max_bytes == max_bytes &&
+                    last.counts == counts && last.lengths == lengths;
   if (!same) {
     last.valid = false;
-    last.plan = make_plan(g, counts, lengths);
+    last.plan = make_plan(g, counts, lengths, max_bytes);
     last.g = g;
+    last.max_bytes = max_bytes;
     last.counts = counts;
     last.lengths = lengths;
     last.valid = true;
@@ -1008,7 +1035,7 @@ int xinfer_batched_flash_attention_noalloc(const xinfer_view4 *q, const xinfer_v
   if (int rc = check_blocks(blocks, blocks_stride)) return rc;
   if (g.B == 0 || g.T == 0) return XINFER_OK;
   if (out == nullptr) return XINFER_ERR_ARGUMENT;
-  const Plan plan = cached_plan(g, counts, lengths);
+  const Plan plan = cached_plan(g, counts, lengths, kScratchBytes);
   if (plan.bytes() > kScratchBytes) return XINFER_ERR_SCRATCH;
   // The device address of the static scratch on the current device (never
   // the host-side name of the array).
