@@ -632,8 +632,9 @@ Plan make_plan(const Geometry &g, const std::vector<int32_t> &counts, const std:
 // simulates its dispatch at several split sizes (about 0.36 ms for the
 // batch-8 D = 256 prefill of 2235 tokens); a call whose geometry, counts,
 // lengths and record limit equal the last one's reuses that plan.  A plan depends
-// on nothing else: not on the device, the stream or the tensors' addresses.
-Plan cached_plan(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths,
+// on nothing else: not on the device, the stream or the tensors' addresses.  The
+// reference holds until the thread's next call.
+const Plan &cached_plan(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths,
                  size_t max_bytes = SIZE_MAX) {
   struct Entry {
     bool valid = false;
@@ -674,62 +675,71 @@ int run_plan(const Plan &plan, const Geometry &g, const xinfer_view4 &q, const x
   float *part_ml =
       plan.records ? reinterpret_cast<float *>(static_cast<char *>(workspace) + plan.part_ml_offset())
                    : nullptr;
-  for (Group grp : plan.groups) {
-    for (AttnArgs *a : {&grp.dec, &grp.pre}) {
-      a->q = view_of(q);
-      a->k = view_of(k);
-      a->v = view_of(v);
-      a->out = static_cast<uint16_t *>(const_cast<void *>(out.data));
-      a->o_sb = out.stride[0];
-      a->o_sh = out.stride[1];
-      a->o_st = out.stride[2];
-      a->part_o = part_o;
-      a->part_ml = part_ml;
-      a->scale_log2 = (float)(scale * 1.4426950408889634);
-      a->D = (int32_t)g.D;
-      a->G = G;
-      a->Hkv = (int32_t)g.Hkv;
-      a->T = (int32_t)g.T;
-      a->blocks = blocks;
-      a->blocks_stride = blocks_stride;
-      a->kv_rows = (int32_t)g.B;
-    }
-    grp.dec.total_items = grp.dec_items;
-    grp.pre.total_items = grp.pre_items;
-    grp.dec.arrive_ctr = nullptr;
-    grp.dec.tag = 0;
-    if (!grp.both && grp.dec_fusable && !merge_launch_forced() && decode_merge_in_launch_pays(grp.dec_items) &&
-        xcd_dispatch_round_robin(stream)) {
-      grp.dec.arrive_ctr = reinterpret_cast<uint64_t *>(static_cast<char *>(workspace) + plan.counters_offset());
-      grp.dec.tag = next_launch_tag();
-      grp.dec_merge_items = 0;  // the decode rows are merged in the launch
-    }
+  // What is launched is a copy with the tensors' places filled in (a Group's
+  // tables are 10 KB; of the empty ones nothing is copied).
+  const auto attention_args = [&](const AttnArgs &planned, int items) {
+    AttnArgs a = planned;
+    a.q = view_of(q);
+    a.k = view_of(k);
+    a.v = view_of(v);
+    a.out = static_cast<uint16_t *>(const_cast<void *>(out.data));
+    a.o_sb = out.stride[0];
+    a.o_sh = out.stride[1];
+    a.o_st = out.stride[2];
+    a.part_o = part_o;
+    a.part_ml = part_ml;
+    a.scale_log2 = (float)(scale * 1.4426950408889634);
+    a.D = (int32_t)g.D;
+    a.G = G;
+    a.Hkv = (int32_t)g.Hkv;
+    a.T = (int32_t)g.T;
+    a.blocks = blocks;
+    a.blocks_stride = blocks_stride;
+    a.kv_rows = (int32_t)g.B;
+    a.total_items = items;
+    return a;
+  };
+  const auto merge_args = [&](const MergeArgs &planned, int items) {
+    MergeArgs m = planned;
+    m.out = static_cast<uint16_t *>(const_cast<void *>(out.data));
+    m.o_sb = out.stride[0];
+    m.o_sh = out.stride[1];
+    m.o_st = out.stride[2];
+    m.part_o = part_o;
+    m.part_ml = part_ml;
+    m.D = (int32_t)g.D;
+    m.G = G;
+    m.total_items = items;
+    return m;
+  };
+  for (const Group &grp : plan.groups) {
+    int dec_merge_items = grp.dec_merge_items;
     hipError_t rc = hipSuccess;
     if (grp.both) {
-      rc = launch_attention_both(grp.dec, grp.pre, dp, grp.dec_columns, stream);
+      rc = launch_attention_both(attention_args(grp.dec, grp.dec_items), attention_args(grp.pre, grp.pre_items), dp,
+                                 grp.dec_columns, stream);
     } else {
-      if (grp.dec_items > 0) rc = launch_decode(grp.dec, dp, grp.dec_columns, grp.dec_items, stream);
-      if (rc == hipSuccess && grp.pre_items > 0) rc = launch_prefill(grp.pre, dp, stream);
+      if (grp.dec_items > 0) {
+        AttnArgs a = attention_args(grp.dec, grp.dec_items);
+        if (grp.dec_fusable && !merge_launch_forced() && decode_merge_in_launch_pays(grp.dec_items) &&
+            xcd_dispatch_round_robin(stream)) {
+          a.arrive_ctr = reinterpret_cast<uint64_t *>(static_cast<char *>(workspace) + plan.counters_offset());
+          a.tag = next_launch_tag();
+          dec_merge_items = 0;  // the decode rows are merged in the launch
+        }
+        rc = launch_decode(a, dp, grp.dec_columns, grp.dec_items, stream);
+      }
+      if (rc == hipSuccess && grp.pre_items > 0)
+        rc = launch_prefill(attention_args(grp.pre, grp.pre_items), dp, stream);
     }
     if (rc != hipSuccess) return XINFER_ERR_LAUNCH;
-    grp.dec_merge.total_items = grp.dec_merge_items;
-    grp.pre_merge.total_items = grp.pre_merge_items;
-    for (MergeArgs *m : {&grp.dec_merge, &grp.pre_merge}) {
-      m->out = static_cast<uint16_t *>(const_cast<void *>(out.data));
-      m->o_sb = out.stride[0];
-      m->o_sh = out.stride[1];
-      m->o_st = out.stride[2];
-      m->part_o = part_o;
-      m->part_ml = part_ml;
-      m->D = (int32_t)g.D;
-      m->G = G;
-    }
-    if (grp.dec_merge_items > 0 && grp.pre_merge_items > 0)
-      rc = launch_merge_both(grp.dec_merge, grp.pre_merge, dp, grp.dec_max_splits, grp.pre_max_splits, stream);
-    else if (grp.dec_merge_items > 0)
-      rc = launch_merge(grp.dec_merge, dp, grp.dec_max_splits, stream);
+    if (dec_merge_items > 0 && grp.pre_merge_items > 0)
+      rc = launch_merge_both(merge_args(grp.dec_merge, dec_merge_items), merge_args(grp.pre_merge, grp.pre_merge_items),
+                             dp, grp.dec_max_splits, grp.pre_max_splits, stream);
+    else if (dec_merge_items > 0)
+      rc = launch_merge(merge_args(grp.dec_merge, dec_merge_items), dp, grp.dec_max_splits, stream);
     else if (grp.pre_merge_items > 0)
-      rc = launch_merge(grp.pre_merge, dp, grp.pre_max_splits, stream);
+      rc = launch_merge(merge_args(grp.pre_merge, grp.pre_merge_items), dp, grp.pre_max_splits, stream);
     if (rc != hipSuccess) return XINFER_ERR_LAUNCH;
   }
   return XINFER_OK;
@@ -947,7 +957,7 @@ int xinfer_batched_flash_attention(const xinfer_view4 *q, const xinfer_view4 *k,
   if (int rc = check_blocks(blocks, blocks_stride)) return rc;
   if (g.B == 0 || g.T == 0) return XINFER_OK;
   if (out == nullptr) return XINFER_ERR_ARGUMENT;
-  const Plan plan = cached_plan(g, counts, lengths);
+  const Plan &plan = cached_plan(g, counts, lengths);
   if (int rc = check_workspace(workspace, workspace_bytes, plan.bytes())) return rc;
   return run_plan(plan, g, *q, *k, *v, blocks, blocks_stride, scale, contiguous_output(g, out), workspace,
                   static_cast<hipStream_t>(stream));
@@ -1035,7 +1045,7 @@ int xinfer_batched_flash_attention_noalloc(const xinfer_view4 *q, const xinfer_v
   if (int rc = check_blocks(blocks, blocks_stride)) return rc;
   if (g.B == 0 || g.T == 0) return XINFER_OK;
   if (out == nullptr) return XINFER_ERR_ARGUMENT;
-  const Plan plan = cached_plan(g, counts, lengths, kScratchBytes);
+  const Plan &plan = cached_plan(g, counts, lengths, kScratchBytes);
   if (plan.bytes() > kScratchBytes) return XINFER_ERR_SCRATCH;
   // The device address of the static scratch on the current device (never
   // the host-side name of the array).
@@ -1056,7 +1066,7 @@ int xinfer_batched_flash_attention_out(const xinfer_view4 *q, const xinfer_view4
   if (int rc = check_blocks(blocks, blocks_stride)) return rc;
   if (g.B == 0 || g.T == 0) return XINFER_OK;
   if (int rc = check_output(g, out)) return rc;
-  const Plan plan = cached_plan(g, counts, lengths);
+  const Plan &plan = cached_plan(g, counts, lengths);
   if (int rc = check_workspace(workspace, workspace_bytes, plan.bytes())) return rc;
   return run_plan(plan, g, *q, *k, *v, blocks, blocks_stride, scale, *out, workspace,
                   static_cast<hipStream_t>(stream));
@@ -1078,7 +1088,7 @@ int xinfer_flash_attention(const xinfer_view4 *q, const xinfer_view4 *k, const x
   if (int rc = check_common(*q, *k, *v, scale)) return rc;
   if (out == nullptr) return XINFER_ERR_ARGUMENT;
   std::vector<int32_t> counts(g.B, (int32_t)g.T), lengths(g.B, (int32_t)valid_length);
-  const Plan plan = cached_plan(g, counts, lengths);
+  const Plan &plan = cached_plan(g, counts, lengths);
   if (int rc = check_workspace(workspace, workspace_bytes, plan.bytes())) return rc;
   return run_plan(plan, g, *q, *k, *v, nullptr, 0, scale, contiguous_output(g, out), workspace,
                   static_cast<hipStream_t>(stream));
