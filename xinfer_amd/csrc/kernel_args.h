@@ -4,6 +4,7 @@
 // and no host<->device copy.
 #pragma once
 
+#include <stddef.h>
 #include <stdint.h>
 
 namespace xattn {
@@ -75,10 +76,12 @@ struct MergeArgs {
   const float *part_ml;
   int32_t D, G;
   int32_t total_items;  // query vectors to merge
-  int32_t lane_items;   // merge_both: the first of them have rows of many splits, the others few
   int32_t nrows;
-  MergeRow rows[kMaxRows];
+  MergeRow rows[kMaxRows];  // from byte 64, two to a 64-byte line
+  int32_t lane_items;       // merge_both: the first of the items have rows of many splits, the others few
 };
+
+static_assert(offsetof(MergeArgs, rows) == 64, "a block's first row is one load");
 
 // Graph-capture mode: one launch shape serves every step, because the kernels
 // read each row's query count and KV length from the device copy of the

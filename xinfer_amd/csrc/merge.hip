@@ -110,18 +110,17 @@ __device__ __forceinline__ void fold_and_write(MergeRed<FS, SG> &red, const floa
 // Every argument of a block, loaded in one round trip (see XATTN_PIN_VIEW).
 struct MergeLocals {
   RowLookup<MergeRow> rows;
-  int total_items, lane_items, nrows, D, G;
+  int total_items, nrows, D, G;
   uint16_t *out;
   int64_t o_sb, o_sh, o_st;
   const float *part_o, *part_ml;
   __device__ __forceinline__ explicit MergeLocals(const MergeArgs &a)
-      : total_items(a.total_items), lane_items(a.lane_items), nrows(a.nrows), D(a.D), G(a.G), out(a.out),
-        o_sb(a.o_sb), o_sh(a.o_sh), o_st(a.o_st), part_o(a.part_o), part_ml(a.part_ml) {
+      : total_items(a.total_items), nrows(a.nrows), D(a.D), G(a.G), out(a.out), o_sb(a.o_sb), o_sh(a.o_sh),
+        o_st(a.o_st), part_o(a.part_o), part_ml(a.part_ml) {
     rows.load(a.rows);
     asm volatile(""
-                 : XATTN_PIN_BEGINS(rows), XATTN_PIN_MERGEROW(rows.first), "+s"(total_items), "+s"(lane_items),
-                   "+s"(nrows), "+s"(D), "+s"(G), "+s"(out), "+s"(o_sb), "+s"(o_sh), "+s"(o_st), "+s"(part_o),
-                   "+s"(part_ml));
+                 : XATTN_PIN_BEGINS(rows), XATTN_PIN_MERGEROW(rows.first), "+s"(total_items), "+s"(nrows), "+s"(D),
+                   "+s"(G), "+s"(out), "+s"(o_sb), "+s"(o_sh), "+s"(o_st), "+s"(part_o), "+s"(part_ml));
   }
 };
 
@@ -129,7 +128,7 @@ struct MergeLocals {
 // with host-planned arguments (merge_kernel, merge_both_kernel) and the
 // graph-capture launch that reads them from device memory (merge_dev_kernel).
 template <int DP, int SG, int THREADS, int FS, bool DEV>
-__device__ __forceinline__ void merge_body(const MergeArgs &a, const MergeLocals &l, int block, int first, int end) {
+__device__ __forceinline__ void merge_body(const MergeArgs &a, const MergeLocals &l, unsigned block, int first, int end) {
   constexpr int FC = DP / 4;                         // feature lanes of a vector
   static_assert(SG == 1 ? FS == FC : FS * SG == THREADS, "block shape");
   constexpr int NS = FC / FS;                        // feature slices per vector (SG > 1)
@@ -147,9 +146,9 @@ __device__ __forceinline__ void merge_body(const MergeArgs &a, const MergeLocals
   const int groups = SG > 1 ? (end - first) * NS : (end - first + VPB - 1) / VPB;
   // A grid sized for more groups (device-planned launches) leaves surplus blocks.
   if constexpr (DEV) {
-    if (block / 8 >= (groups + 7) / 8) return;
+    if ((int)(block / 8) >= (groups + 7) / 8) return;
   }
-  const int group = block % 8 * ((groups + 7) / 8) + block / 8;
+  const int group = (int)(block % 8) * ((groups + 7) / 8) + (int)(block / 8);
   const int vec = first + (SG > 1 ? group / NS : group * VPB + vl);
   const int f = SG > 1 ? (group - (vec - first) * NS) * FS + fl : fl;  // feature lane of the vector
   const bool vvalid = vec < end;
@@ -309,10 +308,12 @@ hipError_t launch_merge(const MergeArgs &a, int dp, int max_splits, hipStream_t 
 template <int DP>
 __global__ void __launch_bounds__(kMergeSerialThreads<DP>) merge_both_kernel(const MergeArgs a) {
   constexpr int THREADS = kMergeSerialThreads<DP>, FC = DP / 4;
+  int lane_items = a.lane_items;
   const MergeLocals l(a);
-  const int lane_blocks = (l.lane_items + 7) / 8 * 8, block = blockIdx.x;
-  if (block < lane_blocks) merge_body<DP, THREADS / FC, THREADS, FC, false>(a, l, block, 0, l.lane_items);
-  else merge_body<DP, 1, THREADS, FC, false>(a, l, block - lane_blocks, l.lane_items, l.total_items);
+  asm volatile("" : "+s"(lane_items));
+  const unsigned lane_blocks = (unsigned)(lane_items + 7) / 8 * 8, block = blockIdx.x;
+  if (block < lane_blocks) merge_body<DP, THREADS / FC, THREADS, FC, false>(a, l, block, 0, lane_items);
+  else merge_body<DP, 1, THREADS, FC, false>(a, l, block - lane_blocks, lane_items, l.total_items);
 }
 
 template <int DP>
