@@ -61,3 +61,12 @@ def test_token_counts_against_the_oracle(gpu_ops, batch, tokens, dim, heads, kv_
                 sizes[r, :, positions[r, t]] = np.maximum(sizes[r, :, positions[r, t]], key_terms[r, :, t])
     check(bits(got_k.cpu()), want_k, sizes)
     assert np.array_equal(bits(got_v.cpu()), want_v)
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+@pytest.mark.parametrize("dim,heads,kv_heads", [(64, 70, 9), (128, 32, 8), (256, 16, 4)])
+@pytest.mark.parametrize("batch,tokens", [(1, 3), (383, 1), (3, 128), (1, 385)])
+def test_tasks_spread_over_blocks(gpu_ops, batch, tokens, dim, heads, kv_heads):
+    """More than eight tasks a token: below 384 tokens over several blocks, above in one block's turns."""
+    test_token_counts_against_the_oracle(gpu_ops, batch, tokens, dim, heads, kv_heads)

@@ -22,8 +22,8 @@
 //
 // A row is a (token, projected head): the Hq query heads, then the Hkv key
 // heads, then the Hkv value heads of each token.  LPR = D/8 lanes hold a row,
-// 8 features (16 bytes) each; a block takes one token, and its waves in turn
-// take 64/LPR heads of one kind at a time (a task).  The partner of lane c for
+// 8 features (16 bytes) each; a wave takes 64/LPR heads of one kind at a time (a
+// task), a block one token's tasks or some of them.  The partner of lane c for
 // the rotation is lane c ^ LPR/2 (the other half of the row).  A key or value row
 // is written to the cache only for a real token (t < count_r) whose position lies
 // in [0, C); query rows are written for every token, as the eager sequence
@@ -37,8 +37,9 @@
 // tokens the key and value rows of padded ones are not read.  Against one row per
 // lane group with all of that per lane (16 query and 8 KV heads, D = 128, in
 // graph replays): 8 x 384 tokens of which 391 are real 17.1 -> 11.1 us, 8 x 512
-// real ones 22.0 -> 17.7 us (4.3 TB/s), 512 tokens 5.2 us both, 8 tokens
-// 3.16 -> 3.10 us.
+// real ones 22.0 -> 17.7 us (69 MB: 3.9 TB/s), 512 tokens 4.4 -> 4.1 us, 8 tokens
+// 3.02 -> 2.82 us.  It loses where a token's heads fill few of a wave's lanes (4 query heads
+// and 1 KV head, D = 64: 8 x 512 tokens 4.3 -> 6.4 us).
 #include <algorithm>
 
 #include "device_common.h"
@@ -107,20 +108,31 @@ __device__ __forceinline__ u32x4 norm_rope(const u32x4 &x, const Floats8 &w, con
   return out;
 }
 
-// Tokens from which blocks have 4 waves, which take several tasks each, and skip
-// padded keys and values.  Below, 8 waves start all loads at once, before the
-// position arrives.  (8 against 4 waves: 512 tokens 5.5 / 5.8 us, 1024 tokens at
-// D = 256 10.6 / 11.5; 2048 tokens 12.3 / 11.2, 8 x 384 14.5 / 11.6, 2048 tokens at
-// D = 256 16.6 / 15.8.)
-constexpr int64_t kNormRopeManyTokens = 2048;
+// Blocks by the number of tokens and of a token's tasks.
+//  kSpread, few tokens of more than 4 tasks: one task a wave in blocks of 4 waves.  A
+//   block of more waves starts later, and one of fewer waves than tasks has them wait
+//   for each other (in blocks of 8 waves -> spread: 16 / 4 heads, D = 256, 12 tasks, 1 token
+//   3.15 -> 2.63 us, 77 tokens 3.53 -> 3.02, 255 3.99 -> 3.84; 16 / 8, D = 128, 8 tasks, 77
+//   tokens 3.12 -> 2.99, 192 3.23 -> 3.25, 512 4.07 -> 4.12; 32 / 8, D = 128, 12 tasks, 255
+//   tokens 3.86 -> 3.70, 512 5.46 -> 5.69).
+//  kWhole: a block takes a token, with a wave per task up to 8.
+//  kMany: up to 4 waves take the tasks in turn and skip padded keys and values; with
+//   fewer waves to start they gain more than the loads, begun before the position arrives,
+//   lose (kWhole / kMany: 512 tokens 5.5 / 5.8 us, 1024 tokens at D = 256 10.6 / 11.5; 2048
+//   tokens 12.3 / 11.2, 8 x 384 14.5 / 11.6, 2048 tokens at D = 256 16.6 / 15.8).
+constexpr int64_t kNormRopeWholeTokens = 384, kNormRopeManyTokens = 2048;
 constexpr int kNormRopeGridRows = 65535;
-constexpr int norm_rope_threads(bool many) { return many ? 256 : 512; }
+enum NormRopeMode { kSpread, kWhole, kMany };
+constexpr int norm_rope_waves(NormRopeMode mode) { return mode == kWhole ? 8 : 4; }  // at most
 
-template <int LPR, bool MANY>
-__global__ void __launch_bounds__(norm_rope_threads(MANY), MANY ? 4 : 2) norm_rope_kernel(const NormRopeArgs a) {
+template <int LPR, NormRopeMode MODE>
+__global__ void __launch_bounds__(64 * norm_rope_waves(MODE), MODE == kWhole ? 2 : 4) norm_rope_kernel(const NormRopeArgs a) {
   constexpr int HEADS = 64 / LPR;  // heads of a task
+  constexpr int WAVES = norm_rope_waves(MODE);
   const int lane = threadIdx.x & 63, head = lane / LPR, dc = lane % LPR;
-  const int b = (int)(blockIdx.z * kNormRopeGridRows + blockIdx.y), t = (int)blockIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  // blockIdx.z: further tasks of the token (kSpread), or further rows.
+  const int b = (int)((MODE == kSpread ? 0 : blockIdx.z * kNormRopeGridRows) + blockIdx.y), t = (int)blockIdx.x;
   if (b >= a.B) return;
   // The row's count and the token's position are block-uniform scalar loads.
   typedef const __attribute__((address_space(4))) int32_t *counts_ptr;
@@ -129,13 +141,14 @@ __global__ void __launch_bounds__(norm_rope_threads(MANY), MANY ? 4 : 2) norm_ro
   const int64_t pos = ((positions_ptr)a.positions)[b * a.pos_sb + t * a.pos_st];
   const int count = cu[b + 1] - cu[b];
   const int q_tasks = (a.Hq + HEADS - 1) / HEADS, kv_tasks = (a.Hkv + HEADS - 1) / HEADS;
-  for (int task = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); task < q_tasks + 2 * kv_tasks;
-       task += norm_rope_threads(MANY) / 64) {
+  // A block of fewer waves than WAVES has one for each task.
+  for (int task = (MODE == kSpread ? (int)blockIdx.z * WAVES : 0) + wave; task < q_tasks + 2 * kv_tasks;
+       task += WAVES) {
     const bool query = task < q_tasks, value = task >= q_tasks + kv_tasks;
     const int h = (task - (query ? 0 : (value ? q_tasks + kv_tasks : q_tasks))) * HEADS + head;
     const int heads = query ? a.Hq : a.Hkv;
     const bool real = t < count && pos >= 0 && pos < a.C;
-    if (MANY && !query && !real) break;
+    if (MODE == kMany && !query && !real) break;
     const View &src = query ? a.q : (value ? a.v : a.k);
     // Lanes past the last head repeat it; they write nothing.
     u32x4 out = load16(src.p + b * src.sb + t * src.st + (int64_t)min(h, heads - 1) * src.sh + dc * 8);
@@ -150,18 +163,27 @@ __global__ void __launch_bounds__(norm_rope_threads(MANY), MANY ? 4 : 2) norm_ro
     } else if (real && h < heads) {
       store16((value ? a.cache_value : a.cache_key) + (((int64_t)b * a.Hkv + h) * a.C + pos) * (LPR * 8) + dc * 8, out);
     }
+    if constexpr (MODE == kSpread) break;
   }
+}
+
+template <int LPR, NormRopeMode MODE>
+static void launch_norm_rope_mode(const NormRopeArgs &a, int tasks, hipStream_t stream) {
+  constexpr int WAVES = norm_rope_waves(MODE);
+  // Tokens by rows (no division in the kernel); a grid takes 65535 rows in y.
+  const int rows = std::min(a.B, kNormRopeGridRows);
+  const dim3 grid(a.T, rows, MODE == kSpread ? (tasks + WAVES - 1) / WAVES : (a.B + rows - 1) / rows);
+  hipLaunchKernelGGL((norm_rope_kernel<LPR, MODE>), grid, dim3(64 * std::min(tasks, WAVES)), 0, stream, a);
 }
 
 template <int LPR>
 static void launch_norm_rope_d(const NormRopeArgs &a, hipStream_t stream) {
+  constexpr int HEADS = 64 / LPR;
+  const int tasks = (a.Hq + HEADS - 1) / HEADS + 2 * ((a.Hkv + HEADS - 1) / HEADS);
   const int64_t tokens = (int64_t)a.B * a.T;
-  const bool many = tokens >= kNormRopeManyTokens;
-  // Tokens by rows (no division in the kernel); a grid takes 65535 rows in y.
-  const dim3 grid(a.T, std::min(a.B, kNormRopeGridRows), (a.B + kNormRopeGridRows - 1) / kNormRopeGridRows);
-  const dim3 block(norm_rope_threads(many));
-  if (many) hipLaunchKernelGGL((norm_rope_kernel<LPR, true>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((norm_rope_kernel<LPR, false>), grid, block, 0, stream, a);
+  if (tokens < kNormRopeWholeTokens && tasks > norm_rope_waves(kSpread)) launch_norm_rope_mode<LPR, kSpread>(a, tasks, stream);
+  else if (tokens < kNormRopeManyTokens) launch_norm_rope_mode<LPR, kWhole>(a, tasks, stream);
+  else launch_norm_rope_mode<LPR, kMany>(a, tasks, stream);
 }
 
 hipError_t launch_norm_rope(const NormRopeArgs &a, hipStream_t stream) {
