@@ -48,11 +48,16 @@ using MergeRed = MergeState[SG > 1 ? SG : 1][SG > 1 ? FS : 1];
 constexpr int kMergeSliceLanes = 16;
 constexpr int kMergeSliceSplits = 64;
 
-// Records a lane loads before it folds any: few with one thread for all splits (registers
-// for more waves), all of its splits up to kMergeSliceSplits, else 16.
-constexpr int merge_inflight(int split_lanes, int slices) {
-  return split_lanes == 1 ? 4 : (slices == 1 ? kMergeSliceSplits / split_lanes : 16);
+// Records a lane loads before it folds any (IN): few with one thread for all splits
+// (registers for more waves), all of its splits up to kMergeSliceSplits
+// (merge_inflight), else 16.  Sixteen for head dim 64 as well, whose block past
+// kMergeSliceSplits differs from the one below in nothing else (one KV head's row of
+// 60000 keys, 235 splits, decode and merge: 13.3 us with 4, 12.9 with 16; 40000 keys and
+// 2 heads 13.2 / 12.95; 79 splits 15.9 both).
+constexpr int merge_inflight(int split_lanes) {
+  return split_lanes == 1 ? 4 : kMergeSliceSplits / split_lanes;
 }
+constexpr int kMergeSliceInflight = 16;
 
 constexpr MergeState kMergeStart{-INFINITY, 0.0f, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
 
@@ -127,7 +132,7 @@ struct MergeLocals {
 // Block `block` of those that merge vectors first .. end - 1: shared by the launches
 // with host-planned arguments (merge_kernel, merge_both_kernel) and the
 // graph-capture launch that reads them from device memory (merge_dev_kernel).
-template <int DP, int SG, int THREADS, int FS, bool DEV>
+template <int DP, int SG, int THREADS, int FS, int IN, bool DEV>
 __device__ __forceinline__ void merge_body(const MergeArgs &a, const MergeLocals &l, unsigned block, int first, int end) {
   constexpr int FC = DP / 4;                         // feature lanes of a vector
   static_assert(SG == 1 ? FS == FC : FS * SG == THREADS, "block shape");
@@ -175,9 +180,10 @@ __device__ __forceinline__ void merge_body(const MergeArgs &a, const MergeLocals
   }
 
   const int g = j % G, i = j / G;
-  fold_and_write<FS, SG, merge_inflight(SG, NS)>(red, l.part_o, l.part_ml, o_base, o_step, ml_base, ml_step, mr.nsplit, vvalid && d < D, sg, fl,
-                         l.out + mr.batch * l.o_sb + (int64_t)(h * G + g) * l.o_sh + (int64_t)i * l.o_st + d,
-                         kMergeStart, sg);
+  fold_and_write<FS, SG, IN>(red, l.part_o, l.part_ml, o_base, o_step, ml_base, ml_step, mr.nsplit, vvalid && d < D,
+                             sg, fl,
+                             l.out + mr.batch * l.o_sb + (int64_t)(h * G + g) * l.o_sh + (int64_t)i * l.o_st + d,
+                             kMergeStart, sg);
 }
 
 // Threads of a block with one thread for all splits: 8 vectors per block for
@@ -187,26 +193,26 @@ __device__ __forceinline__ void merge_body(const MergeArgs &a, const MergeLocals
 template <int DP>
 constexpr int kMergeSerialThreads = DP == 256 ? 512 : 256;
 
-template <int DP, int SG, int THREADS, int FS>
+template <int DP, int SG, int THREADS, int FS, int IN>
 __global__ void __launch_bounds__(THREADS) merge_kernel(const MergeArgs a) {
   const MergeLocals l(a);
-  merge_body<DP, SG, THREADS, FS, false>(a, l, blockIdx.x, 0, l.total_items);
+  merge_body<DP, SG, THREADS, FS, IN, false>(a, l, blockIdx.x, 0, l.total_items);
 }
 
-template <int DP, int SG, int THREADS, int FS>
+template <int DP, int SG, int THREADS, int FS, int IN>
 __global__ void __launch_bounds__(THREADS) merge_dev_kernel(const MergeArgs *__restrict__ a) {
   const MergeLocals l(*a);
-  merge_body<DP, SG, THREADS, FS, true>(*a, l, blockIdx.x, 0, l.total_items);
+  merge_body<DP, SG, THREADS, FS, IN, true>(*a, l, blockIdx.x, 0, l.total_items);
 }
 
 // The merge's launch: host arguments `a`, or (DEV) the arguments at `dev`;
 // the grid covers `vectors` query vectors.
-template <int DP, int SG, int THREADS, int FS, bool DEV>
+template <int DP, int SG, int THREADS, int FS, int IN, bool DEV>
 static void launch_merge_kernel(dim3 grid, const MergeArgs &a, const MergeArgs *dev, hipStream_t stream) {
   if constexpr (DEV)
-    hipLaunchKernelGGL((merge_dev_kernel<DP, SG, THREADS, FS>), grid, dim3(THREADS), 0, stream, dev);
+    hipLaunchKernelGGL((merge_dev_kernel<DP, SG, THREADS, FS, IN>), grid, dim3(THREADS), 0, stream, dev);
   else
-    hipLaunchKernelGGL((merge_kernel<DP, SG, THREADS, FS>), grid, dim3(THREADS), 0, stream, a);
+    hipLaunchKernelGGL((merge_kernel<DP, SG, THREADS, FS, IN>), grid, dim3(THREADS), 0, stream, a);
 }
 
 template <int DP, bool DEV>
@@ -217,18 +223,18 @@ static hipError_t launch_merge_d(const MergeArgs &a, const MergeArgs *dev, int m
   if (max_splits <= kMergeSerialSplits) {
     constexpr int THREADS = kMergeSerialThreads<DP>;
     constexpr int VPB = THREADS / FC;
-    launch_merge_kernel<DP, 1, THREADS, FC, DEV>(dim3(((vectors + VPB - 1) / VPB + 7) / 8 * 8), a, dev, stream);
+    launch_merge_kernel<DP, 1, THREADS, FC, merge_inflight(1), DEV>(dim3(((vectors + VPB - 1) / VPB + 7) / 8 * 8), a, dev, stream);
   } else if (max_splits <= kMergeSliceSplits) {
     // One block per vector: a lane loads its splits in one batch.
-    launch_merge_kernel<DP, 256 / FC, 256, FC, DEV>(dim3((vectors + 7) / 8 * 8), a, dev, stream);
+    launch_merge_kernel<DP, 256 / FC, 256, FC, merge_inflight(256 / FC), DEV>(dim3((vectors + 7) / 8 * 8), a, dev, stream);
   } else {
     // One block per (vector, slice of FS feature lanes).
     constexpr int FS = FC < kMergeSliceLanes ? FC : kMergeSliceLanes;
     const dim3 grid((vectors * (FC / FS) + 7) / 8 * 8);
-    if (max_splits <= 16 * (256 / FS))
-      launch_merge_kernel<DP, 256 / FS, 256, FS, DEV>(grid, a, dev, stream);
+    if (max_splits <= kMergeSliceInflight * (256 / FS))
+      launch_merge_kernel<DP, 256 / FS, 256, FS, kMergeSliceInflight, DEV>(grid, a, dev, stream);
     else
-      launch_merge_kernel<DP, 512 / FS, 512, FS, DEV>(grid, a, dev, stream);
+      launch_merge_kernel<DP, 512 / FS, 512, FS, kMergeSliceInflight, DEV>(grid, a, dev, stream);
   }
   return hipGetLastError();
 }
@@ -312,8 +318,10 @@ __global__ void __launch_bounds__(kMergeSerialThreads<DP>) merge_both_kernel(con
   const MergeLocals l(a);
   asm volatile("" : "+s"(lane_items));
   const unsigned lane_blocks = (unsigned)(lane_items + 7) / 8 * 8, block = blockIdx.x;
-  if (block < lane_blocks) merge_body<DP, THREADS / FC, THREADS, FC, false>(a, l, block, 0, lane_items);
-  else merge_body<DP, 1, THREADS, FC, false>(a, l, block - lane_blocks, lane_items, l.total_items);
+  if (block < lane_blocks)
+    merge_body<DP, THREADS / FC, THREADS, FC, merge_inflight(THREADS / FC), false>(a, l, block, 0, lane_items);
+  else
+    merge_body<DP, 1, THREADS, FC, merge_inflight(1), false>(a, l, block - lane_blocks, lane_items, l.total_items);
 }
 
 template <int DP>
