@@ -1,10 +1,10 @@
 """The decode launch's own merge of split rows against the merge launch.
 
-For decode launches whose split rows have at most eight splits and whose KV
-heads number a multiple of 8, the planner (capi.cpp: decode_merge_fusable,
-choose_decode_rounds, decode_launch_us) lets the last split of each (row, kv
-head) fold the records inside the decode launch, on the XCD where all of that
-group's splits ran (decode.hip: merge_in_launch), instead of a merge launch.
+For decode launches of at most 512 items whose split rows have at most eight
+splits, whose KV heads number a multiple of 8 and whose fold is short, the planner
+(capi.cpp: merge_in_launch_pays) lets the last split of each (row, kv head) fold
+the records inside the decode launch, on the XCD where all of that group's splits
+ran (decode_item.h: merge_in_launch), instead of a merge launch.
 The fold reproduces merge.hip's one-thread-per-(vector, 4 features) layout and
 arithmetic, so the outputs must not depend on the path.
 
@@ -39,8 +39,7 @@ pytestmark = pytest.mark.gpu
 ROOT = Path(__file__).resolve().parents[1]
 
 # (name, Hq, Hkv, D, counts, lengths, capacity, path the planner takes).
-# Keys per one-round item: 128 for head dim 128 with 1-4 query vectors per KV
-# head, 256 for head dim 64, 64 for head dim 256 and for 8 query vectors.
+# Keys per pass of an item: 256, 128, 64 for (padded) head dims 64, 128, 256.
 CASES = [
     ("cfg1_shape", 16, 8, 128, [1], [1024], 4096, "in_launch"),          # 8 splits per kv head
     ("dim64_row", 16, 8, 64, [1], [1000], 2048, "in_launch"),           # 4 splits
@@ -49,12 +48,24 @@ CASES = [
     ("rows_g1_empty", 8, 8, 128, [1, 1, 0, 1], [1024, 5, 3, 300], 2048, "in_launch"),
     ("group4_two_queries", 32, 8, 128, [2, 1, 2], [500, 512, 130], 1024, "in_launch"),  # 8 query vectors
     ("eight_short_rows", 16, 8, 128, [1] * 8, [1024, 1000, 900, 800, 700, 129, 64, 1], 2048, "in_launch"),
-    # cfg3 seed 3's lengths: four-round items (512 keys) bring the longest
+    # cfg3 seed 3's lengths: items of four passes (512 keys) bring the longest
     # row to 7 splits, and the cost model takes them with the in-launch merge.
     ("cfg3_seed3_lengths", 16, 8, 128, [1] * 8, [20, 116, 3394, 53, 3006, 1084, 63, 322], 4096, "in_launch"),
     # Past eight splits, and KV heads not a multiple of 8: the merge launch.
     ("nine_splits", 16, 8, 128, [1], [1100], 2048, "merge"),
     ("four_kv_heads", 16, 4, 128, [1], [1024], 2048, "merge"),
+    # Rows of 9 to 32 query vectors: one and two column groups, up to eight rounds
+    # of the fold; many vectors of many splits go to the merge launch.
+    ("nine_vectors", 24, 8, 128, [3], [1000], 1024, "in_launch"),                          # 8 splits
+    ("sixteen_vectors", 16, 8, 128, [8, 5], [1000, 900], 1024, "in_launch"),               # 8 and 8
+    ("twelve_vectors_d256", 16, 8, 256, [6, 6, 6], [500, 480, 300], 512, "in_launch"),     # 8, 8 and 5
+    ("thirty_two_vectors_d64", 16, 8, 64, [16, 3], [2000, 1500], 2048, "in_launch"),       # 8 and 6
+    ("thirty_two_vectors_d256", 32, 8, 256, [8] * 16, [420] * 16, 512, "in_launch"),       # 2
+    ("long_fold", 32, 8, 256, [8], [380], 512, "merge"),                                   # 6 splits
+    # Beside split prefill rows that fill the chip, in a launch of their own: the merge
+    # launch then serves the prefill rows alone.
+    ("beside_prefill", 16, 8, 128, [1] * 6 + [512] * 2, [1500, 1400, 1300, 1200, 1100, 1000] + [4000] * 2, 4096,
+     "beside_prefill"),
 ]
 
 CHILD = textwrap.dedent(
@@ -152,7 +163,8 @@ def test_in_launch_merge_equals_the_merge_launch(gpu_ops, tmp_path):
         log(f"decode merge paths: {name} ({path})")
         kernels = default_report[name]["kernels"]
         assert any("decode_kernel" in kernel for kernel in kernels), kernels
-        assert ("merge_kernel" in " ".join(kernels)) == (path == "merge"), (name, kernels)
+        assert ("merge_kernel" in " ".join(kernels)) == (path != "in_launch"), (name, kernels)
+        assert ("prefill_kernel" in " ".join(kernels)) == (path == "beside_prefill"), (name, kernels)
         assert "merge_kernel" in " ".join(forced_report[name]["kernels"]), name
         out = default[name]
         assert torch.equal(out.view(torch.int16), forced[name].view(torch.int16)), name

@@ -20,7 +20,7 @@ CALLS = (
     (32, 4, 128, [6, 0, 1, 4, 5, 8, 4, 431, 0, 4, 2, 1, 7, 5],
      [237, 1814, 1814, 1817, 1602, 1499, 1817, 2244, 1814, 1817, 237, 21, 350, 146]),
     (32, 8, 128, [189, 4], [5211, 5026]),
-    (24, 8, 128, [6, 2, 6, 5, 2, 6, 420], [39, 491, 2397, 71, 2393, 2397, 2811]),
+    (32, 4, 128, [0, 4, 1, 0, 2, 1, 395, 4, 4, 2], [715, 1821, 10707, 150, 1434, 3296, 9910, 2794, 178, 351]),
 )
 
 

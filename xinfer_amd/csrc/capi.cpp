@@ -29,7 +29,6 @@ namespace xattn {
 namespace {
 
 constexpr int kCaptureDecodeMaxVectors = 8;  // graph capture: G * T at or below this takes the decode kernel
-constexpr int64_t kDecodeManyItems = 640;  // one-pass decode items from which items are sized to the chip
 constexpr int kPrefillTileQ = 128;         // query vectors per prefill work item
 constexpr int64_t kPrefillMinSplitKeys = 512;
 
@@ -76,7 +75,7 @@ struct Group {
   // differ (a thread folds a few splits, a row of lanes many).
   MergeArgs dec_merge{}, pre_merge{};
   int dec_merge_items = 0, pre_merge_items = 0, pre_max_splits = 1;
-  // The decode launch may merge its split rows itself (decode_merge_fusable).
+  // The decode launch may merge its split rows itself (merge_in_launch_pays).
   bool dec_fusable = false;
   bool both = false;  // decode and prefill rows in one launch (one_launch_pays)
 };
@@ -104,120 +103,151 @@ constexpr double kMergeLaunchUs = 5.0;
 constexpr double kRecordBytesPerUs = 5.0e6;
 constexpr int kCusPerXcd = 32;
 
-// Decode merge choice.  The merge launch after a decode kernel costs an
-// empty kernel's time there (1.8-2.1 us measured on MI355X) plus the cold
-// round trip of its records (2-2.5 us).  The in-launch merge makes every
-// block wait, before it retires, for its record stores and one counter round
-// trip (kArrivalUs), which delays the blocks queued behind it once per wave of
-// resident blocks, and leaves the last split of each (row, kv head) a fold at
-// the tail (kInLaunchFoldUs).  Resident decode blocks: 256 CUs x 2 (64 KB of
-// each CU's 160 KB of LDS per block).
-constexpr double kDecodeMergeLaunchUs = 4.0;
-constexpr double kArrivalUs = 1.5;
-constexpr double kInLaunchFoldUs = 1.0;
-constexpr int64_t kDecodeResidentBlocks = 512;
-// Decode kernel latency model: a launch floor, then whichever is longer of
-// streaming the KV bytes and the rounds of the items each resident block
-// runs one after another.
-constexpr double kDecodeFloorUs = 2.0;
-constexpr double kDecodeBytesPerUs = 5.5e6;
-constexpr double kDecodeRoundUs = 1.2;
+// Decode merge choice.  The merge launch costs an empty kernel's time and the cold
+// round trips of its records, four splits at a time up to kMergeSerialSplits, and of
+// the records themselves, written and read.
+constexpr double kDecodeRecordBytesPerUs = 3.0e6;
+double merge_launch_us(int64_t splits, double record_bytes) {
+  return (splits <= kMergeSerialSplits ? 2.0 + (double)ceil_div(splits, 4) : 4.5) + record_bytes / kDecodeRecordBytesPerUs;
+}
+// The in-launch merge makes every block wait, before it retires, for its record
+// stores and one counter round trip, and leaves the last split of each (row, kv head)
+// a fold at the tail, in rounds of the 256 quads of features its threads take at a
+// time.  So it does not pay for many vectors of many splits.  Measured on MI355X, one
+// row, 8 KV heads, D = 128, in the launch / by the merge launch: 8 splits of 8, 16, 32
+// vectors 8.8 / 10.5, 9.2 / 9.8, 12.7 / 11.4 us, 3 splits of 32 10.2 / 9.5; D = 256: 5 splits of
+// 16 10.8 / 10.4, 6 of 32 16.2 / 13.2; 16 rows, 2 splits of 32 vectors, D = 256: 22.5 / 25.3.
+double merge_in_launch_us(int64_t splits, int64_t vectors, int dp) {
+  return 1.5 + (double)ceil_div(vectors * (dp / 4), 64 * kDecodeWaves) * (0.05 + 0.12 * (double)splits);
+}
+// Resident decode blocks: 256 CUs x 2 (66 to 80 KB of each CU's 160 KB of LDS per
+// block).  A launch of more would make its blocks wait more than once.
+constexpr int64_t kDecodeResidentBlocks = 2 * kDecodeCus;
 
-// Modelled time of a decode launch and its merge: `items` blocks of `rounds`
-// rounds over kv_bytes; split: some row has several splits, merged in the
-// launch (in_launch) or by the merge launch.
-double decode_launch_us(int64_t items, int rounds, double kv_bytes, bool split, bool in_launch) {
-  const double waves = (double)ceil_div(items, kDecodeResidentBlocks);
-  double us = kDecodeFloorUs + std::max(kv_bytes / kDecodeBytesPerUs, rounds * kDecodeRoundUs * waves);
-  if (split) us += in_launch ? kArrivalUs * waves + kInLaunchFoldUs : kDecodeMergeLaunchUs;
+// Whether a decode launch merges its own split rows.  Only with Hkv a multiple of 8 (the
+// kernel gives XCD x the kv heads h = x mod 8 of every row) and at most
+// kMergeSerialSplits splits a row, the merge layout the in-launch fold reproduces.
+bool merge_in_launch_pays(int64_t Hkv, int64_t items, int64_t splits, int64_t vectors, double record_bytes, int dp) {
+  return Hkv % 8 == 0 && items <= kDecodeResidentBlocks && splits > 1 && splits <= kMergeSerialSplits &&
+         merge_in_launch_us(splits, vectors, dp) < merge_launch_us(splits, record_bytes);
+}
+
+// Modelled time of a decode launch and its merge, without what no choice of items
+// changes.  A CU alone with an item takes kDecodePassUs for a pass (64 KB at 45 GB/s),
+// two items on it take as long as both in turn; HBM serves all CUs at
+// kDecodeSharePassUs a pass each.  Past the resident blocks, CUs take items as they come
+// free: most of a longest item is left at the end, and every item's start counts.
+constexpr double kDecodePassUs = 1.5, kDecodeSharePassUs = 1.8;
+struct DecodeRow {
+  uint32_t passes, vectors;
+};
+struct DecodeLoad {
+  std::array<DecodeRow, kMaxRows> rows;  // in launch order
+  int n = 0;
+  int64_t passes = 0;  // of all (row, kv head) pairs
+};
+double decode_us(const Geometry &g, const DecodeLoad &load, int dp, int64_t m) {
+  int64_t items = 0, splits = 1, vectors = 0, records = 0, longest = 0, paired = 0;
+  for (int r = 0; r < load.n; ++r) {
+    const uint32_t passes = load.rows[r].passes, nsplit = (passes + (uint32_t)m - 1) / (uint32_t)m;
+    const int64_t size = nsplit == 1 ? passes : (passes + nsplit - 1) / nsplit;
+    longest = std::max(longest, size);
+    const int64_t next = items + g.Hkv * nsplit;
+    if (items <= kDecodeCus && kDecodeCus < next) paired = size;  // shares the CU of the first item
+    items = next;
+    if (nsplit > 1) {
+      splits = std::max<int64_t>(splits, nsplit);
+      vectors = std::max<int64_t>(vectors, load.rows[r].vectors);
+      records += g.Hkv * nsplit * load.rows[r].vectors;
+    }
+  }
+  // One item a CU leaves HBM a little idle while it starts and ends (decode of 8 rows,
+  // 126 MB: 27.1 us with 240 items, 26.8 with 512).
+  const double share =
+      (items <= kDecodeCus ? 1.02 : 1.0) * kDecodeSharePassUs * (double)load.passes / kDecodeCus;
+  double us = items <= kDecodeResidentBlocks
+                  ? std::max(kDecodePassUs * (double)(longest + paired), share)
+                  : std::max(kDecodePassUs * (double)longest, share) + 0.75 * kDecodePassUs * (double)longest +
+                        0.75 * (double)items / kDecodeResidentBlocks;
+  if (splits > 1) {
+    const double bytes = (double)(records * (4 * g.D + 8));
+    us += merge_in_launch_pays(g.Hkv, items, splits, vectors, bytes, dp) ? merge_in_launch_us(splits, vectors, dp)
+                                                                        : merge_launch_us(splits, bytes);
+  }
   return us;
 }
 
-// The in-launch merge pays when its block waits and tail fold cost less
-// than the merge launch.
-bool decode_merge_in_launch_pays(int64_t items) {
-  return kArrivalUs * (double)ceil_div(items, kDecodeResidentBlocks) + kInLaunchFoldUs < kDecodeMergeLaunchUs;
-}
-
-// Keys per decode item of rows [row0, row0 + nrows), in whole passes of a
-// block's four waves (decode_tokens_per_item).
+// Passes of a block's four waves (decode_tokens_per_item) per decode item.
 //
-// Launches with at least kDecodeManyItems one-pass items (sized against one-pass
-// items, attention alone: 1400 of them 19.8 / 24.4 us, 1304 19.4 / 23.0, 1520 21.7 / 25.1,
-// about 1000 15.5 / 17.0, D = 256, 700, 14.7 / 18.2; 32 rows of up to 700 keys, about 800,
-// 13.2 / 12.7), and those with rows of
-// more than kExactVectors query vectors (whose records are large) or beside
-// prefill rows, size their items to the chip (sized; kernel_args.h: kDecodeCus).
-// Smaller launches compare, by decode_launch_us, items of one pass against items
-// of kDecodeItemRounds passes when those bring every split row within eight
-// splits (fusable: Hkv a multiple of 8 and no split prefill row in the launch);
-// longer items trade latency for the merge launch.  Measured on MI355X (cfg3
-// seeds 1 and 3, one pass + merge launch against four passes + in-launch merge):
-// 10.2 / 11.9 us and 13.6 / 12.8 us; the model picks the faster of each.
-// vectors: rows of up to that many query vectors per KV head are decode rows.
-// stretch: items that many times as long (make_plan: fewer records).
-struct DecodeChoice {
-  bool sized;
-  int64_t keys;
-};
-DecodeChoice choose_decode(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths,
-                           int64_t row0, int nrows, int G, int dp, int64_t vectors, bool fusable, int64_t stretch) {
-  int64_t items[2] = {0, 0}, max_splits[2] = {1, 1}, keys = 0, widest = 0, longest = 1, pairs = 0;
-  bool prefill = false;
-  const int64_t pass = decode_tokens_per_item(dp);
-  const int rounds[2] = {1, kDecodeItemRounds};
-  std::array<int64_t, kMaxRows> passes;
-  int n = 0;
-  for (int r = 0; r < nrows; ++r) {
-    const int64_t qv = (int64_t)counts[row0 + r] * G, len = lengths[row0 + r];
-    prefill = prefill || qv > vectors;
-    if (qv <= 0 || qv > vectors) continue;
-    widest = std::max(widest, qv);
-    keys += g.Hkv * len;
-    pairs += g.Hkv;
-    passes[n++] = ceil_div(len, pass);
-    longest = std::max(longest, ceil_div(len, pass));
-    for (int o = 0; o < 2; ++o) {
-      const int64_t splits = ceil_div(len, rounds[o] * pass);
-      items[o] += g.Hkv * splits;
-      max_splits[o] = std::max(max_splits[o], splits);
-    }
+// By decode_us, launches of at most one one-pass item per CU take items of one pass or of
+// kDecodeItemRounds.  Others, and those with rows of more than kExactVectors query vectors
+// (whose records are large), choose among the fewest passes that leave one item per
+// CU, two, four or eight, those that bring every row within the merge in the
+// launch, and no split.  Measured on MI355X against all numbers of passes, 287
+// launches of 1-64 rows (uniform and log-uniform lengths up to 16384 keys; 16 / 8 and 32 / 8
+// heads of 128, 8 / 8 of 64, 16 / 4 of 256): 2% above the best on average; 7.5% with
+// one item per CU or two by evenness, four where neither was even, whose merge launch
+// that rule did not count (32 rows of up to 1000 keys, D = 128: 20.6 us, now 15.5; 32
+// of up to 700, 928 one-pass items, 19.5, now 14.1).
+//
+// Beside prefill rows, where the decode items are merged by a launch, the evenness
+// rule (kernel_args.h: kDecodeCus) stays: 7 decode rows and 384 tokens, D = 128, in one
+// launch 21.0 us with it, 24.1 with the few items that decode_us prefers.
+int64_t choose_decode_passes(const Geometry &g, const DecodeLoad &load, int dp, bool prefill) {
+  int64_t longest = 1, widest = 0, pairs = g.Hkv * load.n;
+  for (int r = 0; r < load.n; ++r) {
+    longest = std::max<int64_t>(longest, load.rows[r].passes);
+    widest = std::max<int64_t>(widest, load.rows[r].vectors);
   }
-  if (items[0] >= kDecodeManyItems || widest > kExactVectors || prefill) {
-    // The fewest passes per item that leave at most `limit` items.
-    auto least = [&](int64_t limit) {
-      auto fits = [&](int64_t m) {  // items only fall as m grows
-        int64_t count = 0;
-        for (int r = 0; r < n; ++r) count += ((uint32_t)passes[r] + (uint32_t)m - 1) / (uint32_t)m;
-        return g.Hkv * count <= std::max(limit, pairs);
-      };
-      int64_t low = std::max<int64_t>(1, ceil_div(items[0], limit)), high = low;
-      for (int64_t step = 1; high < longest && !fits(high); step *= 2) {
-        low = high + 1;
-        high = std::min(longest, high + step);
-      }
-      while (low < high) {
-        const int64_t m = (low + high) / 2;
-        if (fits(m)) high = m;
-        else low = m + 1;
-      }
-      return low;
+  // The fewest passes per item, from `low`, that leave at most `limit` items.
+  auto least = [&](int64_t limit, int64_t low) {
+    auto fits = [&](int64_t passes) {  // items only fall as the passes grow
+      int64_t count = 0;
+      for (int r = 0; r < load.n; ++r) count += (load.rows[r].passes + (uint32_t)passes - 1) / (uint32_t)passes;
+      return g.Hkv * count <= std::max(limit, pairs);
     };
-    auto even = [&](int64_t m, int64_t limit) { return m * limit * kDecodeEvenDen <= items[0] * kDecodeEvenNum; };
-    const int64_t m1 = least(kDecodeCus), m2 = least(2 * kDecodeCus);
-    int64_t m = 2 * m2 < m1 ? m2 : m1;
-    if (!even(m1, kDecodeCus) && !even(m2, 2 * kDecodeCus)) m = least(4 * kDecodeCus);
-    return {true, m * pass * stretch};
+    low = std::max(low, ceil_div(load.passes, limit));
+    int64_t high = low;
+    for (int64_t step = 1; high < longest && !fits(high); step *= 2) {
+      low = high + 1;
+      high = std::min(longest, high + step);
+    }
+    while (low < high) {
+      const int64_t mid = (low + high) / 2;
+      if (fits(mid)) high = mid;
+      else low = mid + 1;
+    }
+    return low;
+  };
+  if (prefill) {
+    auto even = [&](int64_t m, int64_t limit) { return m * limit * kDecodeEvenDen <= load.passes * kDecodeEvenNum; };
+    const int64_t m2 = least(2 * kDecodeCus, 1), m1 = least(kDecodeCus, m2);
+    if (!even(m1, kDecodeCus) && !even(m2, 2 * kDecodeCus)) return least(4 * kDecodeCus, 1);
+    return 2 * m2 < m1 ? m2 : m1;
   }
-  if (!fusable || max_splits[1] > kMergeSerialSplits) return {false, pass * stretch};
-  const double kv_bytes = 4.0 * (double)(keys * g.D);
-  double us[2];
-  for (int o = 0; o < 2; ++o) {
-    const bool split = max_splits[o] > 1;
-    const bool in_launch = max_splits[o] <= kMergeSerialSplits && decode_merge_in_launch_pays(items[o]);
-    us[o] = decode_launch_us(items[o], rounds[o], kv_bytes, split, in_launch);
+  int64_t best = 1;
+  double best_us = INFINITY;
+  auto consider = [&](int64_t m) {
+    const double us = decode_us(g, load, dp, m);
+    if (us < best_us) {
+      best_us = us;
+      best = m;
+    }
+  };
+  if (load.passes <= kDecodeCus && widest <= kExactVectors) {
+    consider(1);
+    consider(kDecodeItemRounds);
+    return best;
   }
-  return {false, (us[1] < us[0] ? kDecodeItemRounds : 1) * pass * stretch};
+  int64_t m = 0;
+  for (int64_t limit = 8 * kDecodeCus; limit >= kDecodeCus; limit /= 2) {
+    const int64_t next = std::min(least(limit, std::max<int64_t>(m, 1)), longest);
+    if (next > m) consider(next);
+    m = next;
+  }
+  if (g.Hkv % 8 == 0) consider(ceil_div(longest, kMergeSerialSplits));
+  if (m < longest) consider(longest);
+  return best;
 }
 
 // 64-key tiles of prefill item (split, query tile) of row rs: the key range
@@ -398,17 +428,6 @@ int64_t choose_split_keys(const Geometry &g, const std::vector<int32_t> &counts,
   return best_keys;
 }
 
-// Whether a group's decode launch can merge its own split rows: Hkv is a
-// multiple of 8 (the kernel gives XCD x the kv heads h = x mod 8 of every row),
-// and every split row has at most kMergeSerialSplits splits, the merge layout
-// the in-launch fold reproduces.  More splits, or vectors, make the fold at the
-// launch's tail longer than a merge launch, which spreads it over the chip
-// (measured on MI355X: 12 vectors of up to 11 splits 53.8 us against 29.5 + 4.6,
-// 2 vectors of up to 12 splits 28.4 against 22.8 + 4.5).
-bool decode_merge_fusable(const Group &grp, int64_t Hkv) {
-  return grp.dec_items > 0 && grp.dec_merge_items > 0 && Hkv % 8 == 0 && grp.dec_max_splits <= kMergeSerialSplits;
-}
-
 // Whether this device deals consecutive blocks to its 8 XCDs in turn, probed
 // once per device.  The probe runs on a private non-blocking stream, with
 // this thread in relaxed capture mode, so that neither the caller's stream
@@ -495,6 +514,7 @@ int64_t decode_vector_limit(const Geometry &g, const std::vector<int32_t> &count
 // (0.04), but 6 rows and 4 x 512 tokens 128 -> 131 (0.2), 5 rows and 512 tokens 36.9 -> 39.2
 // (0.9), 7 long rows 45.2 -> 53.5 (1.8), 31 long rows and 4 x 512 tokens 187 -> 211 (0.7);
 // D = 64 109 -> 126 (0.8).
+constexpr double kDecodeBytesPerUs = 5.5e6;
 bool one_launch_pays(const Geometry &g, const AttnArgs &dec, int G, int dp, const std::vector<double> &work) {
   double bytes = 0, total = 0, longest = 0;
   for (int r = 0; r < dec.nrows; ++r) {
@@ -513,7 +533,7 @@ bool one_launch_pays(const Geometry &g, const AttnArgs &dec, int G, int dp, cons
 
 // The schedule of a call whose rows of up to decode_vectors query vectors per KV
 // head take the decode kernel, its items `stretch` times as long as
-// choose_decode has them.
+// choose_decode_passes has them.
 Plan plan_rows(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths,
                int64_t decode_vectors, int64_t stretch) {
   Plan plan;
@@ -528,24 +548,35 @@ Plan plan_rows(const Geometry &g, const std::vector<int32_t> &counts, const std:
     Group grp;
     grp.row0 = (int)row0;
     grp.nrows = (int)std::min<int64_t>(kMaxRows, g.B - row0);
-    bool prefill_split = false;
-    for (int r = 0; r < grp.nrows; ++r) {
-      const int64_t qv = (int64_t)counts[row0 + r] * G;
-      if (qv > decode_vectors && prefill_splits(lengths[row0 + r], split_keys) > 1) prefill_split = true;
-    }
-    const DecodeChoice choice = choose_decode(g, counts, lengths, row0, grp.nrows, G, dp, decode_vectors,
-                                              g.Hkv % 8 == 0 && !prefill_split, stretch);
     int64_t records = 0;  // of this group: the groups' launches run one after another
     // Longer decode rows first: the launch's last items are then short ones.  Prefill
     // rows keep the batch's order, which choose_split_keys simulates (sorted as
     // well, a ragged D = 256 batch took 488 us in place of 457).
-    std::vector<int> order(grp.nrows);
-    std::iota(order.begin(), order.end(), 0);
+    std::array<int, kMaxRows> order;
+    const auto order_end = order.begin() + grp.nrows;
+    std::iota(order.begin(), order_end, 0);
     auto decode_length = [&](int r) {
       return (int64_t)counts[row0 + r] * G <= decode_vectors ? lengths[row0 + r] : 0;
     };
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return decode_length(x) > decode_length(y); });
-    for (const int r : order) {
+    std::sort(order.begin(), order_end, [&](int x, int y) {
+      return decode_length(x) != decode_length(y) ? decode_length(x) > decode_length(y) : x < y;
+    });
+    DecodeLoad load;
+    bool prefill = false;
+    const int64_t pass = decode_tokens_per_item(dp);
+    for (auto r = order.begin(); r != order_end; ++r) {
+      const int64_t qv = (int64_t)counts[row0 + *r] * G;
+      if (qv > decode_vectors) prefill = true;
+      else if (qv > 0) {
+        const int64_t passes = ceil_div(lengths[row0 + *r], pass);
+        load.rows[load.n++] = {(uint32_t)passes, (uint32_t)qv};
+        load.passes += g.Hkv * passes;
+      }
+    }
+    const int64_t item_keys = choose_decode_passes(g, load, dp, prefill) * pass * stretch;
+    int64_t split_vectors = 0, decode_records = 0;  // most vectors of a split decode row
+    for (auto next = order.begin(); next != order_end; ++next) {
+      const int r = *next;
       const int64_t b = row0 + r;
       const int cnt = counts[b], len = lengths[b];
       const int64_t qv = (int64_t)cnt * G;
@@ -558,14 +589,18 @@ Plan plan_rows(const Geometry &g, const std::vector<int32_t> &counts, const std:
       const bool decode = qv <= decode_vectors;  // includes rows with no query (zero fill only)
       if (decode) {
         grp.dec_columns = std::max(grp.dec_columns, decode_column_groups((int)qv));
-        if (cnt > 0) rs.nsplit = (int32_t)ceil_div(len, choice.keys);
+        if (cnt > 0) rs.nsplit = (int32_t)ceil_div(len, item_keys);
         // Equal splits, in whole wave tiles: none is empty, since a split never
-        // holds more than choice.keys, a multiple of them.
+        // holds more than item_keys, a multiple of them.
         const int64_t tile = decode_tokens_per_item(dp) / kDecodeWaves;
         rs.ntiles = (int32_t)(ceil_div(ceil_div(len, rs.nsplit), tile) * tile);
         rs.item_begin = grp.dec_items;
         grp.dec_items += (int)(g.Hkv * rs.nsplit);
         grp.dec_max_splits = std::max(grp.dec_max_splits, (int)rs.nsplit);
+        if (rs.nsplit > 1) {
+          split_vectors = std::max(split_vectors, qv);
+          decode_records += g.Hkv * rs.nsplit * qv;
+        }
       } else {
         rs.ntiles = (int32_t)ceil_div(qv, kPrefillTileQ);
         rs.nsplit = prefill_splits(len, split_keys);
@@ -593,7 +628,8 @@ Plan plan_rows(const Geometry &g, const std::vector<int32_t> &counts, const std:
       a.rows[a.nrows++] = rs;
     }
     plan.records = std::max(plan.records, records);
-    grp.dec_fusable = decode_merge_fusable(grp, g.Hkv) && !(prefill_split && !choice.sized);
+    grp.dec_fusable = merge_in_launch_pays(g.Hkv, grp.dec_items, grp.dec_max_splits, split_vectors,
+                                           (double)(decode_records * (4 * g.D + 8)), dp);
     if (grp.dec_fusable) plan.counters = std::max<int64_t>(plan.counters, grp.dec_items);
     if (grp.pre_items > 0) {
       const std::vector<double> work = prefill_item_work(grp.pre.rows, grp.pre.nrows, g.Hkv, G, dp);
@@ -721,8 +757,7 @@ int run_plan(const Plan &plan, const Geometry &g, const xinfer_view4 &q, const x
     } else {
       if (grp.dec_items > 0) {
         AttnArgs a = attention_args(grp.dec, grp.dec_items);
-        if (grp.dec_fusable && !merge_launch_forced() && decode_merge_in_launch_pays(grp.dec_items) &&
-            xcd_dispatch_round_robin(stream)) {
+        if (grp.dec_fusable && !merge_launch_forced() && xcd_dispatch_round_robin(stream)) {
           a.arrive_ctr = reinterpret_cast<uint64_t *>(static_cast<char *>(workspace) + plan.counters_offset());
           a.tag = next_launch_tag();
           dec_merge_items = 0;  // the decode rows are merged in the launch

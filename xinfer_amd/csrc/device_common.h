@@ -282,8 +282,9 @@ __device__ __forceinline__ void capture_row(const CaptureArgs &c, int r, int &co
 
 
 // Splits of row `lane` of a graph-capture decode launch (every lane of the wave
-// calls it): the host planner's choice (capi.cpp: choose_decode) from the
-// device lengths, with a coarser search.  Items take whole passes of a block, at
+// calls it), from the device lengths: the evenness rule (kernel_args.h: kDecodeCus)
+// with a coarse search; every captured launch is merged by a launch, so what a merge in the
+// launch would save does not enter.  Items take whole passes of a block, at
 // least c.pass_min; there are never more than 4 * kDecodeCus + the (row, kv head)
 // pairs, and no row takes more than c.splits_max splits (the records hold those).
 __device__ __forceinline__ int capture_splits(const CaptureArgs &c, int lane, int count, int length) {
