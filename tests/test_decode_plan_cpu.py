@@ -36,3 +36,10 @@ def test_items_and_merge(lib, name, counts, lengths, heads, kv_heads, dim, passe
     counters = kv_heads * sum(splits) if in_launch else 0
     assert decode_workspace(lib, counts, lengths, heads, kv_heads, dim, 16384) == expected_workspace(records, dim,
                                                                                                       counters)
+
+
+def test_rows_on_both_sides_of_the_multiplied_division(lib):  # noqa: F811
+    """34 million keys: 2^19 passes at head dim 256, where the planner goes on to divide."""
+    for passes in ((1 << 19) - 5, (1 << 19) + 5):
+        length = 64 * passes
+        assert decode_workspace(lib, [1], [length], 1, 1, 256, length) == expected_workspace(512, 256, 0)

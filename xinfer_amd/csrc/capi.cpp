@@ -145,11 +145,29 @@ struct DecodeLoad {
   std::array<DecodeRow, kMaxRows> rows;  // in launch order
   int n = 0;
   int64_t passes = 0;  // of all (row, kv head) pairs
+  int64_t longest = 1, widest = 0;  // row's passes, row's vectors
 };
+// ceil(passes / m) by a multiplication: 2^40 / m rounded up is exact for passes and m
+// below 2^19 (33 million keys), where it is used; a plan of 32 rows takes some 800 of them.
+class SplitCount {
+ public:
+  SplitCount(int64_t m, int64_t longest)
+      : m_((uint32_t)m), inverse_(longest < (1 << 19) && m < (1 << 19) ? ((uint64_t(1) << 40) - 1) / m_ + 1 : 0) {}
+  uint32_t operator()(uint32_t passes) const {
+    const uint32_t n = passes + m_ - 1;
+    return inverse_ ? (uint32_t)((n * inverse_) >> 40) : n / m_;
+  }
+
+ private:
+  uint32_t m_;
+  uint64_t inverse_;
+};
+
 double decode_us(const Geometry &g, const DecodeLoad &load, int dp, int64_t m) {
+  const SplitCount split_count(m, load.longest);
   int64_t items = 0, splits = 1, vectors = 0, records = 0, longest = 0, paired = 0;
   for (int r = 0; r < load.n; ++r) {
-    const uint32_t passes = load.rows[r].passes, nsplit = (passes + (uint32_t)m - 1) / (uint32_t)m;
+    const uint32_t passes = load.rows[r].passes, nsplit = split_count(passes);
     const int64_t size = nsplit == 1 ? passes : (passes + nsplit - 1) / nsplit;
     longest = std::max(longest, size);
     const int64_t next = items + g.Hkv * nsplit;
@@ -194,16 +212,13 @@ double decode_us(const Geometry &g, const DecodeLoad &load, int dp, int64_t m) {
 // rule (kernel_args.h: kDecodeCus) stays: 7 decode rows and 384 tokens, D = 128, in one
 // launch 21.0 us with it, 24.1 with the few items that decode_us prefers.
 int64_t choose_decode_passes(const Geometry &g, const DecodeLoad &load, int dp, bool prefill) {
-  int64_t longest = 1, widest = 0, pairs = g.Hkv * load.n;
-  for (int r = 0; r < load.n; ++r) {
-    longest = std::max<int64_t>(longest, load.rows[r].passes);
-    widest = std::max<int64_t>(widest, load.rows[r].vectors);
-  }
+  const int64_t longest = load.longest, pairs = g.Hkv * load.n;
   // The fewest passes per item, from `low`, that leave at most `limit` items.
   auto least = [&](int64_t limit, int64_t low) {
-    auto fits = [&](int64_t passes) {  // items only fall as the passes grow
+    auto fits = [&](int64_t m) {  // items only fall as m grows
+      const SplitCount split_count(m, longest);
       int64_t count = 0;
-      for (int r = 0; r < load.n; ++r) count += (load.rows[r].passes + (uint32_t)passes - 1) / (uint32_t)passes;
+      for (int r = 0; r < load.n; ++r) count += split_count(load.rows[r].passes);
       return g.Hkv * count <= std::max(limit, pairs);
     };
     low = std::max(low, ceil_div(load.passes, limit));
@@ -234,7 +249,7 @@ int64_t choose_decode_passes(const Geometry &g, const DecodeLoad &load, int dp, 
       best = m;
     }
   };
-  if (load.passes <= kDecodeCus && widest <= kExactVectors) {
+  if (load.passes <= kDecodeCus && load.widest <= kExactVectors) {
     consider(1);
     consider(kDecodeItemRounds);
     return best;
@@ -571,6 +586,8 @@ Plan plan_rows(const Geometry &g, const std::vector<int32_t> &counts, const std:
         const int64_t passes = ceil_div(lengths[row0 + *r], pass);
         load.rows[load.n++] = {(uint32_t)passes, (uint32_t)qv};
         load.passes += g.Hkv * passes;
+        load.longest = std::max(load.longest, passes);
+        load.widest = std::max(load.widest, qv);
       }
     }
     const int64_t item_keys = choose_decode_passes(g, load, dp, prefill) * pass * stretch;
