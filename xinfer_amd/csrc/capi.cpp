@@ -102,6 +102,8 @@ constexpr double kPrefillItemUs = 4.5;
 constexpr double kMergeLaunchUs = 5.0;
 constexpr double kRecordBytesPerUs = 5.0e6;
 constexpr int kCusPerXcd = 32;
+// Prefill items that leave a quarter of the CUs free.
+constexpr int kPrefillFreeItems = 8 * kCusPerXcd * 3 / 4;
 
 // Decode merge choice.  The merge launch costs an empty kernel's time and the cold
 // round trips of its records, four splits at a time up to kMergeSerialSplits, and of
@@ -494,24 +496,42 @@ uint64_t next_launch_tag() {
 
 // Query vectors per KV head up to which a row of the call takes the decode
 // kernel: kStreamMaxVectors, whose columns hold them and whose stream is bound by
-// HBM; but kExactVectors, as far as the weights' precision needs it, where a
-// decode launch would serve only a few keys of rows with more beside prefill
-// rows.  Measured on MI355X: prompts of 77, 201 and 13 tokens (one vector each,
-// D = 64) 13.4 us in one launch, 17.6 with the 13-token row in its own; eight rows
-// of 2-6 tokens (12 vectors) over 39000 keys 73 us with the prefill kernel's
-// 128-vector tiles, 36 with this one.
-constexpr int64_t kShortRowKeys = 32768;  // keys of all KV heads
+// HBM; but kExactVectors, as far as the weights' precision needs it, where prefill rows
+// are there and a decode launch would serve only rows with more, in two cases.  Head
+// dim 64, whose prefill items take little (0.9 us a tile): unless the prefill rows'
+// items leave CUs free (one_launch_pays) and some row is longer than kShortRowKeys.  Head dims
+// to 128 with at most two query heads per KV head: if no row is longer than
+// kPrefillMinSplitKeys, where no prefill row is split and merged.  Measured on MI355X, short
+// rows of 9-32 vectors on the decode / the prefill kernel:
+// D = 64: beside 200 tokens, 1, 4, 12 rows of 32 keys 9.2 / 7.6, 9.3 / 7.7, 9.7 / 8.2 us, of 700 12.4 /
+//  12.0, 13.1 / 12.5, 15.1 / 13.4, of 6000 14.3 / 14.5, 21.7 / 25.3, 40.1 / 46.8; beside 384 of 1400 keys
+//  12 rows of 700 17.2 / 23.4; beside 812 tokens over 5000 keys (288 items) 4 rows of 32, 700,
+//  6000 keys 24.7 / 24.1, 33.7 / 24.0, 41.1 / 32.9.
+// D = 128, 2 heads: beside 200 tokens 1, 4, 12 rows of 200 keys 13.0 / 12.3, 14.1 / 12.7, 16.3 / 13.5,
+//  of 700 14.5 / 16.8, 15.7 / 17.2, 21.2 / 29.0; beside 384 tokens 4 rows of 32 17.9 / 28.0;
+//  beside 812 tokens 12 rows of 32 54.8 / 65.2, but 4 of 700 56.3 / 50.0.  4 heads: beside 200
+//  tokens 4 rows of 200 keys 14.8 / 15.7.
+// D = 256: beside 200 tokens 4 rows of 32 17.6 / 20.2, beside 384 12 of 32 32.2 / 62.9.
+constexpr int64_t kShortRowKeys = 1024;
 int64_t decode_vector_limit(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths,
                             int G) {
   bool narrow = false, wide = false;
-  int64_t keys = 0;
+  int64_t longest = 0, prefill_items = 0;  // of kPrefillMinSplitKeys keys
   for (int64_t r = 0; r < g.B; ++r) {
     const int64_t qv = (int64_t)counts[r] * G;
-    if (qv > kStreamMaxVectors) wide = true;
-    else if (qv > kExactVectors) keys += g.Hkv * lengths[r];
-    else if (qv > 0) narrow = true;
+    if (qv > 0) longest = std::max<int64_t>(longest, lengths[r]);
+    if (qv > kStreamMaxVectors) {
+      wide = true;
+      prefill_items += g.Hkv * ceil_div(qv, kPrefillTileQ) * ceil_div(lengths[r], kPrefillMinSplitKeys);
+    } else if (qv > 0 && qv <= kExactVectors) {
+      narrow = true;
+    }
   }
-  return wide && !narrow && keys <= kShortRowKeys ? kExactVectors : kStreamMaxVectors;
+  if (!wide || narrow) return kStreamMaxVectors;
+  bool decode = true;
+  if (g.D <= 64) decode = prefill_items <= kPrefillFreeItems && longest > kShortRowKeys;
+  else if (g.D <= 128 && G <= 2) decode = longest > kPrefillMinSplitKeys;
+  return decode ? kStreamMaxVectors : kExactVectors;
 }
 
 // Whether the decode rows `dec` and the prefill rows whose items take `work`
@@ -542,7 +562,7 @@ bool one_launch_pays(const Geometry &g, const AttnArgs &dec, int G, int dp, cons
     longest = std::max(longest, us);
   }
   const double prefill_us = std::max(longest, total / (8.0 * kCusPerXcd));
-  const bool free_cus = work.size() <= 8 * kCusPerXcd * 3 / 4;
+  const bool free_cus = work.size() <= kPrefillFreeItems;
   return bytes / kDecodeBytesPerUs <= (free_cus ? (dp == 128 ? 1.0 : 2.6) : 0.1) * prefill_us;
 }
 
