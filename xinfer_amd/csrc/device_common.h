@@ -48,15 +48,6 @@ __device__ __forceinline__ u32x4 load16(const uint16_t *p) {
 }
 __device__ __forceinline__ void store16(uint16_t *p, u32x4 v) { *as_global(reinterpret_cast<u32x4 *>(p)) = v; }
 
-// 4-term bf16 dot product of two 8-element bf16 vectors accumulated in fp32.
-__device__ __forceinline__ float dot8_bf16(u32x4 a, u32x4 b, float acc) {
-  acc = __builtin_amdgcn_fdot2_f32_bf16(as_bf16x2(a.x), as_bf16x2(b.x), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(as_bf16x2(a.y), as_bf16x2(b.y), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(as_bf16x2(a.z), as_bf16x2(b.z), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(as_bf16x2(a.w), as_bf16x2(b.w), acc, false);
-  return acc;
-}
-
 // DPP lane move within a 16-lane row (gfx9 encodings).
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float x) {
@@ -88,7 +79,6 @@ __device__ __forceinline__ float pair_max32(float x) {
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 constexpr int kDppRowRor8 = 0x128;    // lane i <- lane (i + 8) mod 16 within each row
-constexpr int kDppRowRor4 = 0x124;    // lane i <- lane (i + 4) mod 16 within each row
 
 // All-reduce (sum) over aligned groups of N lanes, N in {8,16,32,64}.  Every lane
 // of a group ends with the same value (each level adds a pair of equal partials).
@@ -100,68 +90,6 @@ __device__ __forceinline__ float group_sum(float x) {
   if constexpr (N >= 16) x += dpp_move<kDppMirror>(x);
   if constexpr (N >= 32) x = pair_sum16(x);
   if constexpr (N >= 64) x += __shfl_xor(x, 32);
-  return x;
-}
-
-
-// Reductions over the lanes l, l + S, l + 2S, ... (S = stride, a power of two
-// >= 8): the key-row slots of a wave in the decode kernel.
-template <int S>
-__device__ __forceinline__ float slot_sum(float x) {
-  if constexpr (S <= 8) x += dpp_move<kDppRowRor8>(x);
-  if constexpr (S <= 16) x = pair_sum16(x);
-  if constexpr (S <= 32) x = pair_sum32(x);
-  return x;
-}
-template <int S>
-__device__ __forceinline__ float slot_max(float x) {
-  if constexpr (S <= 8) x = fmaxf(x, dpp_move<kDppRowRor8>(x));
-  if constexpr (S <= 16) x = pair_max16(x);
-  if constexpr (S <= 32) x = pair_max32(x);
-  return x;
-}
-
-// Reduce-scatter of QR (2 or 4) per-lane partial dot products over aligned
-// groups of N (16 or 32) lanes: lane l ends with the group's full sum for
-// query l & (QR - 1).  The first log2(QR) steps halve the values each lane
-// keeps (DPP xor 1, xor 2); the rest all-reduce over the lanes of one query
-// with symmetric steps (xor 2 for QR = 2, rotate 8 then rotate 4 within the
-// 16-lane row, the permlane16 pair), so those lanes end with equal sums.
-template <int QR, int N>
-__device__ __forceinline__ float rs_sum(const float (&d)[QR], int lane) {
-  static_assert((QR == 2 || QR == 4) && (N == 16 || N == 32), "reduce-scatter shape");
-  const bool b0 = lane & 1;
-  float v;
-  if constexpr (QR == 4) {
-    const float k0 = b0 ? d[1] : d[0], k1 = b0 ? d[3] : d[2];
-    const float s0 = b0 ? d[0] : d[1], s1 = b0 ? d[2] : d[3];
-    const float n0 = k0 + dpp_move<kDppXor1>(s0), n1 = k1 + dpp_move<kDppXor1>(s1);
-    const bool b1 = lane & 2;
-    const float kk = b1 ? n1 : n0, ss = b1 ? n0 : n1;
-    v = kk + dpp_move<kDppXor2>(ss);
-  } else {
-    const float k0 = b0 ? d[1] : d[0], s0 = b0 ? d[0] : d[1];
-    v = k0 + dpp_move<kDppXor1>(s0);
-    v += dpp_move<kDppXor2>(v);
-  }
-  v += dpp_move<kDppRowRor8>(v);
-  v += dpp_move<kDppRowRor4>(v);
-  if constexpr (N == 32) v = pair_sum16(v);
-  return v;
-}
-// Value of query J from the lane of the quad that holds it (after rs_sum).
-template <int QR, int J>
-__device__ __forceinline__ float quad_query(float x) {
-  constexpr int ctrl = QR == 4 ? J * 0x55 : (J == 0 ? 0xA0 : 0xF5);
-  return dpp_move<ctrl>(x);
-}
-
-__device__ __forceinline__ float wave_max(float x) {
-  for (int m = 32; m >= 1; m >>= 1) x = fmaxf(x, __shfl_xor(x, m));
-  return x;
-}
-__device__ __forceinline__ float wave_sum(float x) {
-  for (int m = 32; m >= 1; m >>= 1) x += __shfl_xor(x, m);
   return x;
 }
 
@@ -183,10 +111,6 @@ __device__ __forceinline__ u32x4 buffer_load16_l2(__amdgpu_buffer_rsrc_t rsrc, u
 }
 __device__ __forceinline__ u32x2 buffer_load8_l2(__amdgpu_buffer_rsrc_t rsrc, uint32_t voffset) {
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, voffset, 0, 1));
-}
-// Non-temporal (cache policy nt) 16-byte load, for data read exactly once.
-__device__ __forceinline__ u32x4 buffer_load16_stream(__amdgpu_buffer_rsrc_t rsrc, uint32_t voffset, uint32_t soffset) {
-  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voffset, soffset, 2));
 }
 
 // Kernel arguments reach a wave through scalar loads from the kernarg

@@ -36,7 +36,7 @@ struct AttnArgs {
   float *part_ml;            // [records][2] (running max in log2 units, sum)
   float scale_log2;          // softmax scale * log2(e)
   int32_t D, G, Hkv, T;
-  int32_t total_items;       // work items of this launch (the decode grid may be smaller)
+  int32_t total_items;       // work items of this launch
   int32_t nrows;
   RowSched rows[kMaxRows];
   // Prefill: items [xcd_begin[x], xcd_begin[x + 1]) run on XCD x (block b

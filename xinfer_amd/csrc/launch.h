@@ -21,10 +21,12 @@ constexpr int kExactVectors = 8;
 constexpr int decode_column_groups(int vectors) {
   return 3 * vectors <= 16 || (vectors > kExactVectors && vectors <= 16) ? 1 : 2;
 }
-// Keys one pass of a decode block's four waves takes for padded head dim `dp`.
+// Passes per decode item of a small launch that takes more than one (capi.cpp:
+// choose_decode_passes, check_capture).
 constexpr int kDecodeItemRounds = 4;
-int decode_tokens_per_item(int dp);
 constexpr int kDecodeWaves = 4;
+// Keys one pass of a decode block's waves takes for padded head dim `dp`.
+int decode_tokens_per_item(int dp);
 hipError_t launch_decode(const AttnArgs &a, int dp, int columns, int items, hipStream_t stream);
 
 hipError_t launch_prefill(const AttnArgs &a, int dp, hipStream_t stream);

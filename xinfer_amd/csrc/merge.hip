@@ -63,11 +63,11 @@ constexpr MergeState kMergeStart{-INFINITY, 0.0f, f32x4{0.0f, 0.0f, 0.0f, 0.0f}}
 
 // Folds records first, first + SG, ... below nsplit of one query vector into st over
 // this thread's 4 features and writes them as bf16 at dst.  Record s: o at
-// part_o + o_base + s * o_step, (m, l) at part_ml + 2 * (ml_base + s * ml_step).  With SG > 1 split lanes
-// per feature group every thread of the block must call it (it synchronises
-// the block); `active` is false for threads past the vectors or features, and
-// f is the thread's feature lane within the block's FS.  Every record of a
-// batch is loaded before any is folded: a lane's splits take
+// part_o + o_base + s * o_step, (m, l) at part_ml + 2 * (ml_base + s * ml_step).
+// With SG > 1 split lanes per feature group every thread of the block must call it
+// (it synchronises the block); `active` is false for threads past the vectors or
+// features, and f is the thread's feature lane within the block's FS.  Every record
+// of a batch is loaded before any is folded: a lane's splits take
 // ceil(nsplit / (SG * INFLIGHT)) memory round trips.
 template <int FS, int SG, int INFLIGHT>
 __device__ __forceinline__ void fold_and_write(MergeRed<FS, SG> &red, const float *part_o, const float *part_ml,
@@ -285,8 +285,8 @@ __global__ void __launch_bounds__(256) merge_capture_kernel(const CaptureArgs c)
   }
   const int g = j % c.G, i = j / c.G;
   fold_and_write<FC, SG, 16>(red, c.part_o, c.part_ml, o_base, o_step, ml_base, ml_step, nsplit, d < c.D, sg, f,
-                         c.out + r * c.o_sb + (int64_t)(h * c.G + g) * c.o_sh + (int64_t)i * c.o_st + d, st,
-                         ahead ? sg + AHEAD * SG : sg);
+                             c.out + r * c.o_sb + (int64_t)(h * c.G + g) * c.o_sh + (int64_t)i * c.o_st + d, st,
+                             ahead ? sg + AHEAD * SG : sg);
 }
 
 hipError_t launch_merge_capture(const CaptureArgs &c, int dp, hipStream_t stream) {

@@ -753,9 +753,8 @@ hipError_t launch_prefill_capture(const PrefillPlanArgs &p, int dp, unsigned blo
   return hipGetLastError();
 }
 
-// Blocks per launch: 8 times the longest XCD run (blocks past their run exit
-// at once).
-// Blocks of a prefill launch: the XCDs take turns.
+// Blocks of a prefill launch: the XCDs take turns, so 8 times the longest XCD run
+// (blocks past their run exit at once).
 static unsigned prefill_blocks(const AttnArgs &a) {
   int longest = 0;
   for (int x = 0; x < 8; ++x) longest = std::max(longest, a.xcd_begin[x + 1] - a.xcd_begin[x]);
