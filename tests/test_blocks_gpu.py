@@ -13,8 +13,8 @@ copied to where the table points (k_moved[r] = k[blocks[r]]); the moved run
 must also pass the float64 oracle's gates.  Cache rows that no row's page
 names are NaN, so a read of the wrong row poisons the output.  Tables: a
 permutation, a repeating table, entries out of [0, B) (clamped into it), and
-a table viewed with a row stride of 2.  Paths: one-round and four-round
-decode, decode rows merged inside the decode launch, prefill at head dims
+a table viewed with a row stride of 2.  Paths: decode items of one
+pass and of several, decode rows merged inside the decode launch, prefill at head dims
 128 and 256 with and without key splits, head dim 64, the [B, T, Hq, D]
 output and the capture-once operator (decode and prefill shapes).  A
 capacity that is not a multiple of 256 ignores the table.
@@ -34,12 +34,15 @@ pytestmark = pytest.mark.gpu
 CASES = (
     ("decode_one_round", 16, 8, 128, [1, 1, 0, 1], [300, 5, 3, 1000], 1024),
     ("decode_four_rounds", 16, 8, 128, [1, 1, 1, 1, 1, 1, 1, 1],
-     [3000, 2900, 3100, 2500, 3500, 2800, 3300, 3200], 4096),  # 1544 one-round items: four rounds
+     [3000, 2900, 3100, 2500, 3500, 2800, 3300, 3200], 4096),  # 1544 passes in items of 7
     ("decode_merged_in_launch", 16, 8, 128, [1, 1], [1024, 900], 2048),
     ("decode_dim256", 16, 4, 256, [1, 1, 1], [4000, 100, 2048], 4096),
     ("prefill_dim128", 16, 8, 128, [100, 37, 64], [600, 37, 2000], 2048),
     ("prefill_dim256", 16, 4, 256, [60, 130], [500, 1300], 1536),
     ("mixed_dim64", 8, 4, 64, [1, 40, 1], [500, 300, 20], 512),
+    # Decode and prefill rows in one launch (both with key splits) at the other head dims.
+    ("mixed_dim128", 16, 8, 128, [1, 100, 1, 1], [2000, 1400, 20, 700], 2048),
+    ("mixed_dim256", 16, 4, 256, [1, 60, 1, 2], [1300, 1500, 20, 700], 1536),
 )
 
 

@@ -1,16 +1,16 @@
-"""Decode launches whose items take several rounds of keys.
+"""Decode launches whose items take several passes of a block's four waves.
 
-The planner gives decode items four rounds of keys when one-round items
-would number at least 1536 (capi.cpp, make_plan): the block loads and
-computes one round at a time, folds the rounds with one rescale each, masks
-only the waves whose keys reach the row's end or a query's causal limit, and
-writes one output or split record per item.  These cases reach that regime
-with rows of one and two queries (the causal limit then differs between a
-row's query vectors), rows with no query, lengths that leave the last item
-one, two or four rounds long, ending in a partial round, and head dims
-padded to 128 and 256.  Keys past each row's length and queries past its count are
-NaN, so a read outside them poisons the output.  Each result is checked
-against the float64 oracle, and a repeat must be bit-identical.
+A launch with more one-pass items than CUs sizes its items by what it and its merge
+cost (capi.cpp, choose_decode_passes); a row's splits then take equal runs of keys in
+whole wave tiles.  A wave takes every fourth tile of the item through its two LDS
+buffers, masks the tiles that reach the row's end or a query's causal limit, and the
+block writes one output or split record per item.  These cases have items of 5 to 7
+passes, merged by a launch (21 to 36 splits) or in the launch (4 and 6), rows of one
+and two queries (the causal limit then differs between a row's query vectors), rows
+with no query, last splits that end in a partial tile, and head dims padded to 64,
+128 and 256.  Keys past each row's length and queries past its count are NaN, so a
+read outside them poisons the output.  Each result is checked against the float64
+oracle, and a repeat must be bit-identical.
 """
 
 import numpy as np
@@ -23,27 +23,21 @@ from xinfer_amd.attention import batched_attention_metadata
 
 pytestmark = pytest.mark.gpu
 
-# (name, Hq, Hkv, D, counts, lengths, capacity).  One-round items per KV head
-# and row are ceil(L / keys per round): 256 keys for padded dim 64 and 128 for
-# padded dim 128 with up to four query vectors, 32 for padded dim 256 with
-# eight.
+# (name, Hq, Hkv, D, counts, lengths, capacity).  A pass takes 256, 128, 64 keys at
+# padded dims 64, 128, 256 (a wave's tile is a quarter of it).
 CASES = (
-    # 8 KV heads x (125 + 94 + 71) = 2320 one-round items; rows of two queries.
+    # 8 KV heads x (125 + 94 + 71) = 2320 passes in items of 5; rows of two queries.
     ("two_queries_d128", 16, 8, 128, [2, 1, 2, 0], [16000, 12000, 9000, 5], 16384),
-    # Head dim 72 (padded to 128); last items of 129, 1 and 385 keys: two
-    # rounds, one, and four, each ending in a partial round.
+    # Head dim 72 (padded to 128); rows that end one key into a tile, items of 5 passes.
     ("odd_dim_72", 16, 8, 72, [1, 1, 1, 1], [12929, 12801, 12673, 200], 13056),
-    # Head dim 200 (padded to 256), GQA group 4 and two queries: 8 query
-    # vectors per KV head, the widest decode group (32 keys per round);
-    # 4 x (500 + 250 + 65) = 3260 one-round items.
+    # Head dim 200 (padded to 256), GQA group 4 and two queries: 8 query vectors
+    # per KV head, the most with fp32 weights; items of 7 passes.
     ("group4_dim200", 16, 4, 200, [2, 1, 1], [16000, 7999, 2049], 16384),
-    # Head dim 64: 256 keys per round, no reduce-scatter of the scores;
-    # 8 x (25 + 28 + 26 + 36 + 24 + 26 + 27) = 1536 one-round items (the
-    # threshold itself), a two-query row, an empty row, partial last rounds.
+    # Head dim 64: 8 x (25 + 28 + 26 + 36 + 24 + 26 + 27) = 1536 passes in items of
+    # up to 7, merged in the launch; a two-query row, an empty row, partial last tiles.
     ("dim64", 16, 8, 64, [1, 2, 1, 1, 0, 1, 1, 1], [6200, 7000, 6500, 9000, 3, 6144, 6401, 6657], 9216),
-    # Head dim 40 (padded to 64), one query vector per KV head (G = 1):
-    # 8 x (25 + 26 + 26 + 27 + 24 + 25 + 25 + 26) = 1632 one-round items;
-    # the row of 6145 keys ends one key into its last round.
+    # Head dim 40 (padded to 64), one query vector per KV head (G = 1): four splits
+    # a row, merged in the launch; the row of 6145 keys ends one key into its last tile.
     ("odd_dim_40_g1", 8, 8, 40, [1] * 8, [6400, 6600, 6500, 6700, 6144, 6145, 6300, 6500], 8192),
 )
 

@@ -10,13 +10,13 @@ equal, bit for bit, the same two operators launched eagerly on a copy of the
 caches, and stay within the oracle gates.  The default operator, whose plan
 comes from host lengths, agrees within the same gates.
 
-Launch shapes covered (capi.cpp, check_capture): the Qwen3 and Qwen3.5
-decode shapes and the head-dim-64 shape take four-round items, one block
-each; the two-token shapes take one-round items with one block per item; the
-64-row batch at capacity 16384 has 65536 one-round items in a grid capped at
-2048 blocks, so every block takes several items in turn (blockIdx.x,
-blockIdx.x + 2048, ...) and reuses its reduction buffers between them.  Query
-vectors per KV head: 2 (Qwen3), 4 (Qwen3.5, two tokens), 1 (head dim 64,
+Launch shapes covered (capi.cpp, check_capture; device_common.h,
+capture_splits): the Qwen3, Qwen3.5 and head-dim-64 shapes' records hold items of at
+least four passes of a block's waves, the two-token shapes' those of one; the 64-row
+batch at capacity 16384 would have 65536 items of one pass, of which the kernels lay
+out at most 1024 + 512 (four per CU and one per row and KV head), one per block, the
+blocks past them exiting; its 1024 query vectors are merged without early loads.
+Query vectors per KV head: 2 (Qwen3), 4 (Qwen3.5, two tokens), 1 (head dim 64,
 G = 1) and 8 (two tokens with G = 4).
 """
 
@@ -52,13 +52,13 @@ SHAPES = {
         [(2, 4096), (1, 77), (2, 1500), (0, 3)],
         [(2, 2), (2, 4000), (1, 1), (2, 640)],
     ]),
-    # Head dim 64, G = 1: 256 keys per round, four-round items.
+    # Head dim 64, G = 1: 256 keys per pass.
     "d64_group1": (8, 8, 64, 1, 8192, [
         [(1, 8192), (1, 5000), (1, 1), (1, 257), (0, 9), (1, 1024), (1, 3333), (1, 7777)],
         [(1, 3), (1, 8191), (1, 600), (1, 6000), (1, 2), (1, 4097), (0, 1), (1, 1025)],
     ]),
-    # 64 rows at capacity 16384: a grid capped at 2048 blocks over up to
-    # 65536 items, with ragged and empty rows.
+    # 64 rows at capacity 16384: a grid of 1536 blocks, where one-pass items would be
+    # 65536; ragged and empty rows.
     "capped_grid_b64": (16, 8, 128, 1, 16384, [
         [(0 if r % 13 == 5 else 1, (r * 2654435761) % 16384 + 1) for r in range(64)],
         [(0 if r % 7 == 3 else 1, 16384 if r % 9 == 0 else (r * 40503) % 3000 + 1) for r in range(64)],
