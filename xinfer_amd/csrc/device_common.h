@@ -203,6 +203,15 @@ __device__ __forceinline__ void capture_row(const CaptureArgs &c, int r, int &co
   count = min(max(cuq[r + 1] - cuq[r], 0), min(c.T, c.C));
   length = min(max(cuk[r + 1] - cuk[r], max(count, 1)), c.C);
 }
+// The same of a block-uniform row, in scalar loads of one round trip.
+__device__ __forceinline__ void capture_row_uniform(const CaptureArgs &c, int r, int &count, int &length) {
+  typedef const __attribute__((address_space(4))) int32_t *offsets_ptr;
+  const offsets_ptr cuq = (offsets_ptr)c.offsets, cuk = cuq + c.B + 1;
+  int q0 = cuq[r], q1 = cuq[r + 1], k0 = cuk[r], k1 = cuk[r + 1];
+  asm volatile("" : "+s"(q0), "+s"(q1), "+s"(k0), "+s"(k1));
+  count = min(max(q1 - q0, 0), min(c.T, c.C));
+  length = min(max(k1 - k0, max(count, 1)), c.C);
+}
 
 
 // Splits of row `lane` of a graph-capture decode launch (every lane of the wave

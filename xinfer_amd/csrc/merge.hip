@@ -256,27 +256,33 @@ __global__ void __launch_bounds__(256) merge_capture_kernel(const CaptureArgs c)
   constexpr int FC = DP / 4, SG = 256 / FC, AHEAD = 4;
   __shared__ MergeRed<FC, SG> red;
   const int tid = threadIdx.x, lane = tid & 63, f = tid % FC, sg = tid / FC, d = f * 4;
-  const int qv_max = c.T * c.G, per_row = c.Hkv * qv_max;
-  const int r = (int)blockIdx.x / per_row, local = (int)blockIdx.x - r * per_row;
-  const int h = local / qv_max, j = local - h * qv_max;
+  const int r = (int)blockIdx.y, qv_max = c.T * c.G, h = (int)blockIdx.x / qv_max, j = (int)blockIdx.x - h * qv_max;
+  int own_count, own_length;
+  capture_row_uniform(c, r, own_count, own_length);
+  // Nothing to merge past the row's queries, and in a row that one least item holds: such
+  // blocks leave on scalar loads of their own row, before the splits of all rows are
+  // worked out (one row of 30 keys: the launch 3.04 us without, 1.72 with).
+  if (j >= own_count * c.G || own_length <= c.pass_min * c.pass_keys) return;  // block-uniform
   const int64_t ml_base = r * c.row_records + (int64_t)h * c.splits_max * qv_max + j, ml_step = qv_max;
   const int64_t o_base = ml_base * c.D + d, o_step = ml_step * c.D;
-  const bool ahead = gridDim.x <= kMergeAheadVectors;
+  const bool ahead = gridDim.x * gridDim.y <= kMergeAheadVectors;
   u32x2 ml[AHEAD];
   f32x4 o[AHEAD];
-  if (ahead && d < c.D) {
+  if (ahead) {
+    // Lanes past the features or the splits load others' records (a branch around a
+    // load would wait for it).
+    const int64_t o_first = ml_base * c.D + min(d, c.D - 4);
 #pragma unroll
-    for (int u = 0; u < AHEAD; ++u)
-      if (sg + u * SG < c.splits_max) {
-        ml[u] = *as_global(reinterpret_cast<const u32x2 *>(c.part_ml + 2 * (ml_base + (sg + u * SG) * ml_step)));
-        o[u] = *as_global(reinterpret_cast<const f32x4 *>(c.part_o + o_base + (sg + u * SG) * o_step));
-      }
+    for (int u = 0; u < AHEAD; ++u) {
+      const int64_t sp = min(sg + u * SG, c.splits_max - 1);
+      ml[u] = *as_global(reinterpret_cast<const u32x2 *>(c.part_ml + 2 * (ml_base + sp * ml_step)));
+      o[u] = *as_global(reinterpret_cast<const f32x4 *>(c.part_o + o_first + sp * o_step));
+    }
   }
   int count = 0, length = 1;
   if (lane < c.B) capture_row(c, lane, count, length);
-  const int splits = capture_splits(c, lane, count, length);
-  const int qrows = __builtin_amdgcn_readlane(count, r) * c.G, nsplit = __builtin_amdgcn_readlane(splits, r);
-  if (j >= qrows || nsplit <= 1) return;  // block-uniform
+  const int nsplit = __builtin_amdgcn_readlane(capture_splits(c, lane, count, length), r);
+  if (nsplit <= 1) return;
   MergeState st = kMergeStart;
   if (ahead && d < c.D) {
 #pragma unroll
@@ -290,7 +296,7 @@ __global__ void __launch_bounds__(256) merge_capture_kernel(const CaptureArgs c)
 }
 
 hipError_t launch_merge_capture(const CaptureArgs &c, int dp, hipStream_t stream) {
-  const dim3 grid(c.B * c.Hkv * c.T * c.G);
+  const dim3 grid(c.Hkv * c.T * c.G, c.B);
   switch (dp) {
     case 64: hipLaunchKernelGGL(merge_capture_kernel<64>, grid, dim3(256), 0, stream, c); break;
     case 128: hipLaunchKernelGGL(merge_capture_kernel<128>, grid, dim3(256), 0, stream, c); break;
