@@ -27,6 +27,13 @@ CASES = [
     (16, 8, 128, [200, 12, 12], [200, 513, 40], ONE),
     (32, 8, 128, [200, 6, 6], [200, 512, 40], ONE),
     (16, 4, 256, [200, 6, 6], [200, 512, 40], ONE),
+    # Rows of 17-32 vectors alone: few keys, and one row of more; up to 16 vectors; head dim 128.
+    (16, 4, 256, [8, 5], [8, 128], PREFILL),
+    (16, 4, 256, [8, 5], [8, 129], {"decode"}),
+    (16, 4, 256, [4, 3], [8, 128], {"decode"}),
+    (8, 8, 64, [32, 20], [48, 20], PREFILL),
+    (8, 8, 64, [32, 20], [49, 20], {"decode"}),
+    (16, 8, 128, [16, 9], [16, 9], {"decode"}),
     # Decode rows beside few prefill items, many of them; beside prefill items that fill the chip.
     (8, 8, 64, [200] + [1] * 4, [200, 3000, 40, 700, 2000], ONE),
     (16, 8, 128, [200] + [1] * 7, [200] + [2000] * 7, ONE),

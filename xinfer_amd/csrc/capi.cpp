@@ -496,9 +496,10 @@ uint64_t next_launch_tag() {
 
 // Query vectors per KV head up to which a row of the call takes the decode
 // kernel: kStreamMaxVectors, whose columns hold them and whose stream is bound by
-// HBM; but kExactVectors, as far as the weights' precision needs it, where prefill rows
-// are there and a decode launch would serve only rows with more, in two cases.  Head
-// dim 64, whose prefill items take little (0.9 us a tile): unless the prefill rows'
+// HBM; but kExactVectors, as far as the weights' precision needs it, in three cases where
+// every decode row has more.  Without prefill rows: if a row fills two column groups, whose
+// combination takes longer than a whole unsplit prefill item, and all keys are few, by
+// shortest_keys.  Beside prefill rows, head dim 64, whose prefill items take little (0.9 us a tile): unless the prefill rows'
 // items leave CUs free (one_launch_pays) and some row is longer than kShortRowKeys.  Head dims
 // to 128 with at most two query heads per KV head: if no row is longer than
 // kPrefillMinSplitKeys, where no prefill row is split and merged.  Measured on MI355X, short
@@ -512,14 +513,19 @@ uint64_t next_launch_tag() {
 //  beside 812 tokens 12 rows of 32 54.8 / 65.2, but 4 of 700 56.3 / 50.0.  4 heads: beside 200
 //  tokens 4 rows of 200 keys 14.8 / 15.7.
 // D = 256: beside 200 tokens 4 rows of 32 17.6 / 20.2, beside 384 12 of 32 32.2 / 62.9.
+// Alone, 32 vectors: D = 256: 4 rows of 9, 68, 208 keys 9.8 / 7.5, 11.5 / 9.1, 13.4 / 13.5, one row of
+//  208 12.6 / 12.9; D = 64: 33, 92, 232 keys 6.1 / 5.8, 6.3 / 6.25, 6.4 / 7.5; D = 128: 17 keys 7.0 / 7.2,
+//  76 7.0 / 7.7.
 constexpr int64_t kShortRowKeys = 1024;
+constexpr int64_t shortest_keys(int64_t D) { return D <= 64 ? 48 : (D <= 128 ? 0 : 128); }
 int64_t decode_vector_limit(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths,
                             int G) {
   bool narrow = false, wide = false;
-  int64_t longest = 0, prefill_items = 0;  // of kPrefillMinSplitKeys keys
+  int64_t widest = 0, longest = 0, prefill_items = 0;  // of kPrefillMinSplitKeys keys
   for (int64_t r = 0; r < g.B; ++r) {
     const int64_t qv = (int64_t)counts[r] * G;
     if (qv > 0) longest = std::max<int64_t>(longest, lengths[r]);
+    widest = std::max(widest, qv);
     if (qv > kStreamMaxVectors) {
       wide = true;
       prefill_items += g.Hkv * ceil_div(qv, kPrefillTileQ) * ceil_div(lengths[r], kPrefillMinSplitKeys);
@@ -527,9 +533,10 @@ int64_t decode_vector_limit(const Geometry &g, const std::vector<int32_t> &count
       narrow = true;
     }
   }
-  if (!wide || narrow) return kStreamMaxVectors;
+  if (narrow) return kStreamMaxVectors;
   bool decode = true;
-  if (g.D <= 64) decode = prefill_items <= kPrefillFreeItems && longest > kShortRowKeys;
+  if (!wide) decode = widest <= 16 || longest > shortest_keys(g.D);
+  else if (g.D <= 64) decode = prefill_items <= kPrefillFreeItems && longest > kShortRowKeys;
   else if (g.D <= 128 && G <= 2) decode = longest > kPrefillMinSplitKeys;
   return decode ? kStreamMaxVectors : kExactVectors;
 }
