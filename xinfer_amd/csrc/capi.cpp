@@ -6,7 +6,7 @@
 // whose keys are split get fp32 partial records in the caller's workspace,
 // combined by a merge launch after the attention kernels or, for decode rows
 // whose launch allows it, by the last split of each (row, kv head) inside the
-// decode launch (decode.hip: merge_in_launch), which folds in the merge
+// decode launch (decode_item.h: merge_in_launch), which folds in the merge
 // launch's order and arithmetic.  The schedule is a function of the shapes and
 // lengths only, never of tensor data, so results are deterministic and each
 // row is isolated from the others' contents.

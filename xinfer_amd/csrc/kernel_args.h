@@ -43,7 +43,7 @@ struct AttnArgs {
   // runs item xcd_begin[b % 8] + b / 8 while below xcd_begin[b % 8 + 1]).
   // The planner cuts the item list into 8 runs of about equal work.
   int32_t xcd_begin[9];
-  // Decode in-launch merge (decode.hip: merge_in_launch); null: split records
+  // Decode in-launch merge (decode_item.h: merge_in_launch); null: split records
   // go to the merge launch.  One 64-bit arrival counter per decode item, the
   // one of a (row, kv head)'s first item serving it; every counter is left at
   // zero when the launch ends.  tag: nonzero, below 2^36, new for every
@@ -106,7 +106,8 @@ struct CaptureArgs {
   int32_t splits_max;        // most splits of a row
 };
 
-// Decode items for a launch that fills the chip: one per CU or two, whichever
+// Decode items beside prefill rows and of captured launches (the others': capi.cpp,
+// choose_decode_passes), where they fill the chip: one per CU or two, whichever
 // leaves the longest item closer to a CU's (half a CU's) even share of the keys;
 // at most four per CU if both leave it more than kDecodeEvenNum / kDecodeEvenDen
 // of that share.  A CU reads at most about 45 GB/s, 1.8 times its share of HBM, so

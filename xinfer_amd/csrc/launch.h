@@ -17,7 +17,7 @@ hipError_t launch_gemv(const GemvArgs &a, bool fp32, bool vec, hipStream_t strea
 constexpr int kStreamMaxVectors = 32;
 constexpr int kExactVectors = 8;
 // 16-column groups of the decode kernel for a row of `vectors` query vectors
-// per KV head: up to 8 take three columns each (decode.hip: exact weights).
+// per KV head: up to 8 take three columns each (decode_common.h: exact weights).
 constexpr int decode_column_groups(int vectors) {
   return 3 * vectors <= 16 || (vectors > kExactVectors && vectors <= 16) ? 1 : 2;
 }

@@ -1,5 +1,5 @@
 // The fold of split records, shared by the merge launch (merge.hip) and the decode
-// launch's own merge (decode.hip), so that both give the same bits.
+// launch's own merge (decode_item.h), so that both give the same bits.
 #pragma once
 
 #include "device_common.h"
