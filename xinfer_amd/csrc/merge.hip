@@ -246,14 +246,17 @@ static hipError_t launch_merge_d(const MergeArgs &a, const MergeArgs *dev, int m
 // it knows its splits; the records' places do not depend on them, so in small
 // launches a lane's first records are loaded beside the lengths, whether its row
 // has them or not (the workspace holds them all): eight layers' captured steps of
-// 8 rows, 128 vectors, 156.4 -> 150.3 us.  Larger launches, whose records past the
+// 8 rows, 128 vectors, 156.4 -> 148.6 us.  Larger launches, whose records past the
 // splits would be a load worth saving (2 KB a split lane; 512 vectors: 8 MB at
 // most), wait.
 constexpr int kMergeAheadVectors = 512;
 
-template <int DP>
+// AHEAD: records of a lane loaded early, as many as a row of the most splits has
+// (1 to 4; loads past them, all of one record, took a captured step of 16 rows at head
+// dim 64 from 69.2 to 70.8 us).
+template <int DP, int AHEAD>
 __global__ void __launch_bounds__(256) merge_capture_kernel(const CaptureArgs c) {
-  constexpr int FC = DP / 4, SG = 256 / FC, AHEAD = 4;
+  constexpr int FC = DP / 4, SG = 256 / FC;
   __shared__ MergeRed<FC, SG> red;
   const int tid = threadIdx.x, lane = tid & 63, f = tid % FC, sg = tid / FC, d = f * 4;
   const int r = (int)blockIdx.y, qv_max = c.T * c.G, h = (int)blockIdx.x / qv_max, j = (int)blockIdx.x - h * qv_max;
@@ -265,26 +268,23 @@ __global__ void __launch_bounds__(256) merge_capture_kernel(const CaptureArgs c)
   if (j >= own_count * c.G || own_length <= c.pass_min * c.pass_keys) return;  // block-uniform
   const int64_t ml_base = r * c.row_records + (int64_t)h * c.splits_max * qv_max + j, ml_step = qv_max;
   const int64_t o_base = ml_base * c.D + d, o_step = ml_step * c.D;
-  const bool ahead = gridDim.x * gridDim.y <= kMergeAheadVectors;
-  u32x2 ml[AHEAD];
-  f32x4 o[AHEAD];
-  if (ahead) {
-    // Lanes past the features or the splits load others' records (a branch around a
-    // load would wait for it).
-    const int64_t o_first = ml_base * c.D + min(d, c.D - 4);
+  u32x2 ml[AHEAD > 0 ? AHEAD : 1];
+  f32x4 o[AHEAD > 0 ? AHEAD : 1];
+  // Lanes past the features or the splits load others' records (a branch around a
+  // load would wait for it).
+  const int64_t o_first = ml_base * c.D + min(d, c.D - 4);
 #pragma unroll
-    for (int u = 0; u < AHEAD; ++u) {
-      const int64_t sp = min(sg + u * SG, c.splits_max - 1);
-      ml[u] = *as_global(reinterpret_cast<const u32x2 *>(c.part_ml + 2 * (ml_base + sp * ml_step)));
-      o[u] = *as_global(reinterpret_cast<const f32x4 *>(c.part_o + o_first + sp * o_step));
-    }
+  for (int u = 0; u < AHEAD; ++u) {
+    const int64_t sp = min(sg + u * SG, c.splits_max - 1);
+    ml[u] = *as_global(reinterpret_cast<const u32x2 *>(c.part_ml + 2 * (ml_base + sp * ml_step)));
+    o[u] = *as_global(reinterpret_cast<const f32x4 *>(c.part_o + o_first + sp * o_step));
   }
   int count = 0, length = 1;
   if (lane < c.B) capture_row(c, lane, count, length);
   const int nsplit = __builtin_amdgcn_readlane(capture_splits(c, lane, count, length), r);
   if (nsplit <= 1) return;
   MergeState st = kMergeStart;
-  if (ahead && d < c.D) {
+  if (d < c.D) {
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u)
       if (sg + u * SG < nsplit) fold(st, __uint_as_float(ml[u].x), __uint_as_float(ml[u].y), o[u]);
@@ -292,15 +292,28 @@ __global__ void __launch_bounds__(256) merge_capture_kernel(const CaptureArgs c)
   const int g = j % c.G, i = j / c.G;
   fold_and_write<FC, SG, 16>(red, c.part_o, c.part_ml, o_base, o_step, ml_base, ml_step, nsplit, d < c.D, sg, f,
                              c.out + r * c.o_sb + (int64_t)(h * c.G + g) * c.o_sh + (int64_t)i * c.o_st + d, st,
-                             ahead ? sg + AHEAD * SG : sg);
+                             sg + AHEAD * SG);
+}
+
+template <int DP>
+static void launch_merge_capture_d(const CaptureArgs &c, hipStream_t stream) {
+  const dim3 grid(c.Hkv * c.T * c.G, c.B), block(256);
+  constexpr int SG = 256 / (DP / 4);
+  if ((int64_t)grid.x * grid.y > kMergeAheadVectors)
+    hipLaunchKernelGGL((merge_capture_kernel<DP, 0>), grid, block, 0, stream, c);
+  else if (c.splits_max <= SG)
+    hipLaunchKernelGGL((merge_capture_kernel<DP, 1>), grid, block, 0, stream, c);
+  else if (c.splits_max <= 2 * SG)
+    hipLaunchKernelGGL((merge_capture_kernel<DP, 2>), grid, block, 0, stream, c);
+  else
+    hipLaunchKernelGGL((merge_capture_kernel<DP, 4>), grid, block, 0, stream, c);
 }
 
 hipError_t launch_merge_capture(const CaptureArgs &c, int dp, hipStream_t stream) {
-  const dim3 grid(c.Hkv * c.T * c.G, c.B);
   switch (dp) {
-    case 64: hipLaunchKernelGGL(merge_capture_kernel<64>, grid, dim3(256), 0, stream, c); break;
-    case 128: hipLaunchKernelGGL(merge_capture_kernel<128>, grid, dim3(256), 0, stream, c); break;
-    default: hipLaunchKernelGGL(merge_capture_kernel<256>, grid, dim3(256), 0, stream, c); break;
+    case 64: launch_merge_capture_d<64>(c, stream); break;
+    case 128: launch_merge_capture_d<128>(c, stream); break;
+    default: launch_merge_capture_d<256>(c, stream); break;
   }
   return hipGetLastError();
 }
