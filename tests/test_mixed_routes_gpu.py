@@ -38,6 +38,8 @@ CASES = [
     (8, 8, 64, [200] + [1] * 4, [200, 3000, 40, 700, 2000], ONE),
     (16, 8, 128, [200] + [1] * 7, [200] + [2000] * 7, ONE),
     (16, 4, 256, [200] + [1] * 20, [200] + [6000] * 20, TWO),
+    (16, 8, 128, [64] + [1] * 8, [64] + [8000] * 8, TWO),
+    (8, 8, 64, [64] + [1] * 8, [64] + [8000] * 8, TWO),
     (16, 8, 128, [512, 300] + [1] * 6, [3000, 2000] + [3000] * 6, TWO),
 ]
 

@@ -544,22 +544,23 @@ int64_t decode_vector_limit(const Geometry &g, const std::vector<int32_t> &count
 // Whether the decode rows `dec` and the prefill rows whose items take `work`
 // microseconds go in one launch, where decode items stream their keys on the CUs
 // that the prefill items leave free or have left.  An item pair per CU streams less
-// well than two independent blocks, so where the prefill items fill the chip it pays only
-// for a few decode rows beside long prefill; where they leave CUs free (kPrefillFreeItems)
-// the second launch and its merge cost more, for head dim 256, whose pairs stream worst,
-// while the decode rows' bytes (keys, and zeros of padded queries) take up to three
-// times as long as the prefill items.  Measured, two launches -> one (us; ratio of the two times):
+// well than two independent blocks, and a CU holds one pair, so where the prefill items
+// fill the chip it pays only for a few decode rows beside long prefill; where they leave CUs
+// free (kPrefillFreeItems) the second launch and its merge cost more, while the decode
+// rows' bytes (keys, and zeros of padded queries) take up to three times as long as
+// the prefill items.  Measured, two launches -> one (us; ratio of the two times):
 // few prefill items: D = 128: 7 decode rows and 384 tokens 33.8 -> 24.5 (0.9), 20 rows and 200
-// tokens 27.7 -> 26.2 (1.5), 45.5 -> 41.5 (3.6), 95.1 -> 90.4 (10), 7 long rows 43.3 -> 46.1 (3.6);
-// D = 64: 20 rows and 200 tokens 27.4 -> 22.1 (1.9), 51.2 -> 46.3 (5.6); D = 256: 7 rows and 200
-// tokens 37.0 -> 24.8 (1.0), 52.2 -> 45.2 (2.8), 20 rows 57.4 -> 48.1 (3.0), 106 -> 110 (7.9), 20 rows
-// and 384 tokens 72.9 -> 76.9 (2.1), 122 -> 140 (5.1).
+// tokens 27.7 -> 26.2 (1.5), 45.5 -> 41.5 (3.6), 7 long rows 43.3 -> 46.1 (3.6), 8 rows and 64
+// tokens 92 -> 98 (17), 24 rows 126 -> 173 (25); D = 64: 20 rows and 200 tokens 27.4 -> 22.1
+// (1.9), 8 long rows 51.9 -> 53.4 (5.9), 24 rows 69.6 -> 89.8 (8.8), but 60 rows 69.5 -> 61.6
+// (8.2); D = 256: 7 rows and 200 tokens 37.0 -> 24.8 (1.0), 52.2 -> 45.2 (2.8), 20 rows 57.4 ->
+// 48.1 (3.0), 106 -> 110 (7.9), 20 rows and 384 tokens 72.9 -> 76.9 (2.1), 122 -> 140 (5.1).
 // Many: D = 128: 4 rows and 4 x 512 tokens 174 -> 162 (0.1), 1 row and 2000 tokens 198 -> 191
 // (0.04), but 6 rows and 4 x 512 tokens 128 -> 131 (0.2), 5 rows and 512 tokens 36.9 -> 39.2
 // (0.9), 7 long rows 45.2 -> 53.5 (1.8), 31 long rows and 4 x 512 tokens 187 -> 211 (0.7);
 // D = 64 109 -> 126 (0.8).
 constexpr double kDecodeBytesPerUs = 5.5e6;
-bool one_launch_pays(const Geometry &g, const AttnArgs &dec, int G, int dp, const std::vector<double> &work) {
+bool one_launch_pays(const Geometry &g, const AttnArgs &dec, int G, const std::vector<double> &work) {
   double bytes = 0, total = 0, longest = 0;
   for (int r = 0; r < dec.nrows; ++r) {
     const RowSched &rs = dec.rows[r];
@@ -572,7 +573,6 @@ bool one_launch_pays(const Geometry &g, const AttnArgs &dec, int G, int dp, cons
   }
   const double prefill_us = std::max(longest, total / (8.0 * kCusPerXcd));
   const bool free_cus = work.size() <= kPrefillFreeItems;
-  if (free_cus && dp <= 128) return true;
   return bytes / kDecodeBytesPerUs <= (free_cus ? 3.0 : 0.1) * prefill_us;
 }
 
@@ -681,7 +681,7 @@ Plan plan_rows(const Geometry &g, const std::vector<int32_t> &counts, const std:
     if (grp.pre_items > 0) {
       const std::vector<double> work = prefill_item_work(grp.pre.rows, grp.pre.nrows, g.Hkv, G, dp);
       xcd_runs(work, grp.pre.xcd_begin);
-      if (grp.dec_items > 0) grp.both = one_launch_pays(g, grp.dec, G, dp, work);
+      if (grp.dec_items > 0) grp.both = one_launch_pays(g, grp.dec, G, work);
     }
     plan.groups.push_back(grp);
   }
