@@ -34,6 +34,13 @@ CASES = [
     (8, 8, 64, [32, 20], [48, 20], PREFILL),
     (8, 8, 64, [32, 20], [49, 20], {"decode"}),
     (16, 8, 128, [16, 9], [16, 9], {"decode"}),
+    # More short rows than the prefill kernel's blocks take at once.
+    (16, 4, 256, [8] * 64, [60] * 64, PREFILL),
+    (16, 4, 256, [8] * 64 + [7], [60] * 65, {"decode"}),
+    (16, 8, 128, [200] + [12] * 24, [200] + [300] * 24, PREFILL),
+    (16, 8, 128, [200] + [12] * 25, [200] + [300] * 25, ONE),
+    (8, 8, 64, [200] + [24] * 25, [200] + [300] * 25, ONE),
+    (8, 8, 64, [512, 300] + [24] * 11, [3000, 2000] + [6000] * 11, {"decode", "prefill"}),
     # Decode rows beside few prefill items, many of them; beside prefill items that fill the chip.
     (8, 8, 64, [200] + [1] * 4, [200, 3000, 40, 700, 2000], ONE),
     (16, 8, 128, [200] + [1] * 7, [200] + [2000] * 7, ONE),

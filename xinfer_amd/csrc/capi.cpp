@@ -516,12 +516,17 @@ uint64_t next_launch_tag() {
 // Alone, 32 vectors: D = 256: 4 rows of 9, 68, 208 keys 9.8 / 7.5, 11.5 / 9.1, 13.4 / 13.5, one row of
 //  208 12.6 / 12.9; D = 64: 33, 92, 232 keys 6.1 / 5.8, 6.3 / 6.25, 6.4 / 7.5; D = 128: 17 keys 7.0 / 7.2,
 //  76 7.0 / 7.7.
+// In each case only while the short rows' prefill items are few (pairs of row and KV head; items
+// of kPrefillMinSplitKeys keys): alone, D = 256, 60 keys, 256 pairs 13.0 / 11.0, 512 18.1 / 21.9, D = 64,
+//  48 keys, 128 pairs 6.6 / 6.1, 512 8.2 / 11.2; beside 200 tokens, 500 keys, 240 pairs D = 128 28.8 /
+//  35.3, D = 64 16.1 / 18.0; D = 64 beside 812 tokens 1152 items 58.0 / 57.7, 2048 73.5 / 78.4, 2880 88 / 113.
 constexpr int64_t kShortRowKeys = 1024;
 constexpr int64_t shortest_keys(int64_t D) { return D <= 64 ? 48 : (D <= 128 ? 0 : 128); }
 int64_t decode_vector_limit(const Geometry &g, const std::vector<int32_t> &counts, const std::vector<int32_t> &lengths,
                             int G) {
   bool narrow = false, wide = false;
-  int64_t widest = 0, longest = 0, prefill_items = 0;  // of kPrefillMinSplitKeys keys
+  int64_t widest = 0, longest = 0, short_pairs = 0;
+  int64_t prefill_items = 0, short_items = 0;  // of kPrefillMinSplitKeys keys
   for (int64_t r = 0; r < g.B; ++r) {
     const int64_t qv = (int64_t)counts[r] * G;
     if (qv > 0) longest = std::max<int64_t>(longest, lengths[r]);
@@ -529,15 +534,19 @@ int64_t decode_vector_limit(const Geometry &g, const std::vector<int32_t> &count
     if (qv > kStreamMaxVectors) {
       wide = true;
       prefill_items += g.Hkv * ceil_div(qv, kPrefillTileQ) * ceil_div(lengths[r], kPrefillMinSplitKeys);
-    } else if (qv > 0 && qv <= kExactVectors) {
+    } else if (qv > kExactVectors) {
+      short_pairs += g.Hkv;
+      short_items += g.Hkv * ceil_div(lengths[r], kPrefillMinSplitKeys);
+    } else if (qv > 0) {
       narrow = true;
     }
   }
   if (narrow) return kStreamMaxVectors;
+  const bool free_cus = prefill_items <= kPrefillFreeItems;
   bool decode = true;
-  if (!wide) decode = widest <= 16 || longest > shortest_keys(g.D);
-  else if (g.D <= 64) decode = prefill_items <= kPrefillFreeItems && longest > kShortRowKeys;
-  else if (g.D <= 128 && G <= 2) decode = longest > kPrefillMinSplitKeys;
+  if (!wide) decode = widest <= 16 || longest > shortest_keys(g.D) || short_pairs > kDecodeCus;
+  else if (g.D <= 64) decode = free_cus ? longest > kShortRowKeys || short_items > kPrefillFreeItems : short_items > 1024;
+  else if (g.D <= 128 && G <= 2) decode = longest > kPrefillMinSplitKeys || short_pairs > kPrefillFreeItems;
   return decode ? kStreamMaxVectors : kExactVectors;
 }
 
